@@ -302,14 +302,18 @@ int mer_hip_expert_batch_f16(int dtype, size_t d_model, size_t d_ff, size_t n_ex
  * mer_hip_moe_forward -- per token out = [x +] sum_i w_i y_i in slot order,
  * zero-weight slots skipped, misses recorded in the device status -- but
  * the routed (token, slot) pairs are grouped by expert on the device, so
- * every expert's weights are read once for all of its tokens and the
- * projections run as int8 MFMA contractions over token tiles of 16.  This
- * is the batched counterpart of routed_expert_matmul_batch_q4
- * (backend/mod.rs:4401-4418) and of the per-pair dispatch loop of
- * forward_moe_resident_cpu (engine.rs:1761-1848) over a prefill batch.
- * Requires d_model and d_ff to be multiples of 64, n_tokens * top_k <=
- * 4096 and table_len <= 4096.  Inputs are held in 24-bit block fixed
- * point (error <= 2^-24 of each 32-element block's maximum). */
+ * every expert's weights are read once per tile of its tokens and the
+ * projections run as MFMA contractions: int8 over tiles of 16 pairs where
+ * experts have few, f16 over tiles of 64 where they have 16 or more on
+ * average (8 for many large experts).  This is the batched counterpart of
+ * routed_expert_matmul_batch_q4 (backend/mod.rs:4401-4418) and of the
+ * per-pair dispatch loop of forward_moe_resident_cpu (engine.rs:1761-1848)
+ * over a prefill batch.  Requires d_model and d_ff to be multiples of 64,
+ * n_tokens * top_k <= 4096 and table_len <= 4096.  Inputs are held in 24-bit
+ * block fixed point (int8; error <= 2^-24 of each 32-element block's
+ * maximum) or as pairs of f16 with one power-of-two scale per vector (error
+ * <= 2^-23 of each element, or 2^-39 of the vector's maximum where that is
+ * more). */
 int mer_hip_moe_grouped(int dtype, size_t d_model, size_t d_ff,
                         size_t n_tokens, size_t top_k,
                         const void *const *d_expert_table, size_t table_len,

@@ -819,19 +819,47 @@ int run_grouped(Workspace &w, int dtype, size_t dm, size_t dff, uint32_t n_token
   p.hblocks = (uint32_t)(dff / 32);
   p.proj_bytes = div_ceil(dm * dff, 32) * block_bytes(dtype);
   p.status = dev.status;
-  // Token tiles hold <= 16 pairs of one expert: at most n_pairs / 16 full
-  // tiles plus one partial tile per distinct expert.
-  const uint32_t max_tiles = p.n_pairs / 16 + (p.n_pairs < table_len ? p.n_pairs : table_len);
+  const uint32_t max_experts = p.n_pairs < table_len ? p.n_pairs : table_len;
+  // Tiles of 64 pairs on f16 MFMA (gbig) from 16 pairs per expert on average,
+  // or 8 where the experts alone give the 512 resident workgroups four
+  // rounds; else the int8 kernel's tiles of 16.  Call us, int8 / f16, at 8
+  // pairs: Qwen3 Q8_0 138 / 158, Mixtral Q4_0 282 / 287, DeepSeek-V3 Q4_0
+  // (4096 workgroups) 1424 / 1119; at 16 pairs: 208 / 207, 434 / 302, 2290 /
+  // 1600; Mixtral under MER_MOE_QMM at 8 and 16: 279 / 331, 433 / 342.
+  const size_t expert_wgs = (size_t)max_experts * div_ceil(2 * dff, 256);
+  const bool big = p.n_pairs >= 16 * max_experts || (p.n_pairs >= 8 * max_experts && expert_wgs >= 2048);
+  p.mode = !big ? kGroupDigits : p.q8act ? kGroupQ8Act : kGroupF16Pair;
+  const uint32_t tile_pairs = big ? 64u : 16u;
+  // Down rows in up to 4 K parts (whole 4-block stages, about 64 blocks or
+  // more) until 2048 workgroups share the launch: 512 run at once, and a short
+  // last round of whole rows idles the chip.  Mixtral Q4_0 down, us with one
+  // part / with parts: 64 tokens 195 / 94, 128 tokens 281 / 119, 2048 tokens
+  // 1200 / 1105 (combine 20 / 33).
+  p.n_parts = 1;
+  p.part_blocks = p.hblocks;
+  if (big) {
+    const uint32_t wgs = (p.n_pairs / tile_pairs + (max_experts + 1) / 2) * (uint32_t)div_ceil(dm, 256);
+    while (p.n_parts < 4 && wgs * p.n_parts < 2048 && p.hblocks >= 128 * p.n_parts) p.n_parts *= 2;
+    p.part_blocks = (uint32_t)div_ceil(p.hblocks, 4 * p.n_parts) * 4;
+    p.n_parts = (uint32_t)div_ceil(p.hblocks, p.part_blocks);
+  }
+  // At most n_pairs / tile_pairs full tiles plus one partial tile per
+  // distinct expert.
+  const uint32_t max_tiles = p.n_pairs / tile_pairs + max_experts;
 
   auto up64 = [](size_t v) { return (v + 63) / 64 * 64; };  // floats; 256-byte aligned regions
   const size_t n_hdr = 64;
   const size_t n_plist = up64(p.n_pairs);
   const size_t n_ok = up64(p.n_pairs);
   const size_t n_tiles = up64((size_t)max_tiles * sizeof(GroupTile) / 4);
-  const size_t n_xg = up64((size_t)n_tokens * p.xblocks * 32);  // 4 k-group records of 8 dwords per block
-  const size_t n_hg = up64((size_t)p.n_pairs * p.hblocks * 32);
-  const size_t n_pa = up64((size_t)p.n_pairs * dm);
-  const size_t total = n_hdr + n_plist + n_ok + n_tiles + n_xg + n_hg + n_pa;
+  const size_t rec = p.mode == kGroupQ8Act ? 16 : 32;  // record dwords per block
+  const size_t n_xg = up64((size_t)n_tokens * p.xblocks * rec);
+  const size_t n_hg = up64((size_t)p.n_pairs * p.hblocks * rec);
+  const size_t n_xs = big ? up64((size_t)n_tokens * p.xblocks) : 0;
+  const size_t n_hs = big ? up64((size_t)p.n_pairs * p.hblocks) : 0;
+  const size_t n_h32 = big ? up64((size_t)p.n_pairs * dff) : 0;
+  const size_t n_pa = up64((size_t)p.n_parts * p.n_pairs * dm);
+  const size_t total = n_h32 + n_hdr + n_plist + n_ok + n_tiles + n_xg + n_hg + n_xs + n_hs + n_pa;
   float *cur = nullptr;
   int rc = ensure_scratch(w, total, &cur);
   if (rc) return rc;
@@ -847,6 +875,12 @@ int run_grouped(Workspace &w, int dtype, size_t dm, size_t dff, uint32_t n_token
   cur += n_xg;
   p.hg = reinterpret_cast<uint32_t *>(cur);
   cur += n_hg;
+  p.xs = cur;
+  cur += n_xs;
+  p.hs = cur;
+  cur += n_hs;
+  p.h32 = cur;
+  cur += n_h32;
   p.partial = cur;
 
   const int fmt = fmt_of(dtype);
@@ -854,7 +888,7 @@ int run_grouped(Workspace &w, int dtype, size_t dm, size_t dff, uint32_t n_token
   int trc;
   hipError_t e;
   if ((trc = timing_begin(STAGE_PREP, st, &tl))) return trc;
-  if ((e = launch_grouped_prep(p, st)) != hipSuccess) return hip_fail(e, MER_ERR_SUBMISSION, "grouping launch");
+  if ((e = launch_grouped_prep(fmt, p, st)) != hipSuccess) return hip_fail(e, MER_ERR_SUBMISSION, "grouping launch");
   if ((trc = timing_end(tl, st))) return trc;
   if ((trc = timing_begin(STAGE_GATE_UP, st, &tl))) return trc;
   if ((e = launch_grouped_proj(fmt, true, p, max_tiles, st)) != hipSuccess)

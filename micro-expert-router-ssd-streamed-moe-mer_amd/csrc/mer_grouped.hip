@@ -3,8 +3,8 @@
 // A prefill-sized batch routes many tokens to the same expert, so each
 // expert's weights can be read once for all of its tokens.  That turns
 // the per-expert work into a real dense contraction: [rows x K] weights by
-// [K x tokens], run on int8 MFMA (v_mfma_i32_16x16x32_i8, K = 32 = one
-// GGUF block).  Reference semantics are those of the decode path: every
+// [K x tokens], run on MFMA one GGUF block (K = 32) at a
+// time.  Reference semantics are those of the decode path: every
 // routed (token, slot) pair computes y = W_down (silu(W_gate x) * (W_up x))
 // (inference.rs:3291-3306 / :3636-3746) and the token's output is
 // [x +] sum_i w_i y_i in slot order (combine_outputs_into,
@@ -12,37 +12,66 @@
 //
 // Launches, all on the caller's stream:
 //   group_kernel   block 0 groups the routed pairs by expert (counting
-//                  sort) and emits token tiles of <= 16 pairs per expert;
-//                  the other blocks quantise x into 24-bit digit records
-//                  (three base-256 planes, below)
-//   proj_kernel<FUSED>  one workgroup per (token tile, 32 rows of d_ff):
-//                  gate and up rows for the tile's tokens, SiLU * up, h
-//                  quantised per 32-element block
-//   proj_kernel<!FUSED> one workgroup per (token tile, 64 rows of d_model):
-//                  down rows -> w_i * y_i per pair
+//                  sort) and emits token tiles of one expert's pairs; the
+//                  other blocks write x's records (below)
+//   gate/up        one workgroup per (token tile, row tile): gate and up rows
+//                  for the tile's tokens, SiLU * up
+//   [hquant]       gbig only: h's records from f32 h
+//   down           one workgroup per (token tile, row tile[, K part]) ->
+//                  w_i * y_i per pair
 //   combine_kernel out[t] = [x +] sum over slots in slot order
 //
-// Numerics.  The weights are int8 (Q8_0 q, or Q4_0 q-8) with one f16
-// scale per 32-weight block.  Each 32-element block b of an input vector
-// (x, or h for the down projection) is held as s_b * v with
-// s_b = max|x_b| / 8355711 and v = round(x / s_b), split into three signed
-// base-256 digits v = v0 + 256 v1 + 65536 v2 (the bytes of v + 0x808080
-// with their top bits flipped).  Per block, MFMA gives the exact int32
-// sums Pk = sum q*vk (|Pk| < 2^19); P1 + 256 P2 is exact in int32, and the
-// block contributes (256 (P1 + 256 P2) + P0) * d_w * s_b, formed in f32,
-// to an f32 accumulator.  The representation error of v is at most 2^-24
-// of the block's largest |x| (an f32 rounding of that element); non-finite
-// inputs give a NaN scale, so NaN propagates.
+// Two projection kernels, by the pairs an expert has on average (run_grouped):
+//   gproj  int8 MFMA, tiles of 16 pairs, for few pairs, where streaming the
+//          weights is everything;
+//   gbig   f16 MFMA, tiles of 64 pairs.
 //
-// Operand layout of v_mfma_i32_16x16x32_i8: lane l holds 8 int8 of A row
-// (l % 16) and of B column (l % 16), covering the same 8 of the block's 32
-// k-indices (chosen by l / 16) in A and B; output lane l holds rows
+// Numerics.  The weights are integers (Q8_0 q, or Q4_0 q-8) with one f16
+// scale per 32-weight block; they are exact in int8 and in f16.
+//
+// gproj: each 32-element block b of an input vector (x, or h for the down
+// projection) is held as s_b * v with s_b = max|x_b| / 8355711 and
+// v = round(x / s_b), split into three signed base-256 digits
+// v = v0 + 256 v1 + 65536 v2 (the bytes of v + 0x808080 with their top bits
+// flipped).  Per block, MFMA gives the exact int32 sums Pk = sum q*vk
+// (|Pk| < 2^19); P1 + 256 P2 is exact in int32, and the block contributes
+// (256 (P1 + 256 P2) + P0) * d_w * s_b, formed in f32, to an f32
+// accumulator.  The representation error of v is at most 2^-24 of the
+// block's largest |x|; non-finite inputs give a NaN scale, so NaN
+// propagates.
+//
+// gbig: an input vector is held as S * (hi + lo) with S a power of two that
+// puts its largest element in [2^14, 2^15), hi the f16 nearest to x / S and
+// lo the f16 nearest to the rest: an error of at most 2^-23 |x|, and 2^-39 of
+// the vector's largest element where lo underflows (elements below 2^-16 of
+// it).  Per block two chained products, lo first, give sum q (hi + lo) in
+// f32; times d_w it goes to an f32 accumulator.  The matrix unit rounds its
+// sums towards minus infinity, a bias that would grow with the number of
+// blocks, so every other block carries both its weights and its scale
+// negated and the biases cancel (Mixtral prefill, 2048 tokens, against
+// float64: 3.6e-7 without, 2.1e-7 with; the int8 kernel 2.6e-7).  Partial
+// sums of 16 blocks are added up in a second accumulator (one accumulator:
+// 4.0e-7, two: 1.7e-7).
+//
+// gbig under MER_MOE_QMM: the activation is Candle's Q8_0, integers of at most
+// 8 bits, exact in one f16; a block's sum is exact in f32 and contributes
+// times d_w * d_x.
+//
+// Operand layout of v_mfma_i32_16x16x32_i8 (gproj): lane l holds 8 int8 of A
+// row (l % 16) and of B column (l % 16), covering the same 8 of the block's
+// 32 k-indices (chosen by l / 16) in A and B; output lane l holds rows
 // 4 (l / 16) + i, i = 0..3, of column l % 16.  Weights are staged through
 // LDS as [row][block][32 int8] (rows padded to spread banks) plus f32
 // scales [block][row]; the input digits are stored per (vector, block) as
 // 4 groups x {8 bytes v0, 8 bytes v1, 8 bytes v2, f32 scale, pad}, so a
 // lane reads the B operands of its k-group and the block scale from one
 // 32-byte record.
+//
+// gbig takes the inputs as A rows and the weights as B columns, so an output
+// lane's column is one weight row and its scale d_w one register.  Weights go
+// to LDS as they are and become f16 in registers.
+#include <type_traits>
+
 #include "mer_internal.hpp"
 
 namespace mer {
@@ -50,7 +79,16 @@ namespace mer {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
+constexpr uint32_t kBigTok = 64;             // pairs per token tile of gbig
+constexpr uint32_t kGMaxRun = 32;            // consecutive work items on one XCD (gbig)
+constexpr uint32_t kNoLoad = 0x80000000u;    // an offset past every buffer: reads zeros
+
+// ---- gproj geometry -----------------------------------------------------
 constexpr uint32_t kGTok = 16;           // pairs per token tile (MFMA N)
 constexpr int kGWavesPerEu = 4;
 // Workgroup geometry: four waves, RT row tiles of 16 rows (RT = 4 or 8),
@@ -74,7 +112,6 @@ struct GGeom {
 };
 constexpr float kGIntMax = 8355711.0f;   // |v| bound (0x7f7f7f): v + 0x808080 stays in 24 bits
 constexpr uint32_t kGRec = 8;            // dwords per (vector, block, k-group) record: 3 digit planes, scale, pad
-constexpr uint32_t kNoChunkG = 0x80000000u;
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 
@@ -88,6 +125,14 @@ __device__ __forceinline__ bool pair_valid(const GroupedParams &p, uint32_t pair
   if (blob) *blob = b;
   return b != nullptr;
 }
+
+// How a call's input vectors are held: records of one k-group (8 elements)
+// of one block.
+enum GMode : int {
+  kDigits = kGroupDigits,  // gproj: three int8 digit planes and the block scale
+  kQ8Act = kGroupQ8Act,    // gbig, QMatMul: Q8_0 integers in f16; one scale per block
+  kF16Pair = kGroupF16Pair // gbig: f16 high and low parts; one scale per vector
+};
 
 // Quantise 8 elements (one MFMA k-group) of a block whose 4 groups sit in
 // 4 adjacent lanes (lane & 3 = group): block max by shuffles, then one
@@ -146,28 +191,128 @@ __device__ __forceinline__ void quant_group(const float (&v)[8], uint32_t *dst, 
   o[1] = make_uint4(d[4], d[5], __float_as_uint(s), 0u);
 }
 
-// Block 0: group the routed pairs by expert.  Other blocks: quantise x.
-__global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
-  if (blockIdx.x > 0) {
-    const uint32_t g = (blockIdx.x - 1) * blockDim.x + threadIdx.x;  // (token, block, group)
-    const uint32_t total = p.n_tok * p.xblocks * 4;
-    // whole quads stay together for the shuffles; quads past the end idle
-    const bool valid = g < total;
-    const uint32_t tb = g / 4, m = g % 4;
+// Element of its block at position i of k-group m of gbig's records.
+// Q4_0: the eight weights of qs dword m in the order unpack_q4 yields them.
+template <int FMT>
+__device__ __forceinline__ constexpr uint32_t kgroup_elem(uint32_t m, int i) {
+  if constexpr (FMT == FMT_Q4_0) {
+    constexpr int o[8] = {0, 2, 16, 18, 1, 3, 17, 19};
+    return 4 * m + o[i];
+  } else {
+    return 8 * m + i;
+  }
+}
+
+// One Q8_0-activation record: 8 elements (in kgroup_elem order) of a block
+// whose 4 groups sit in 4 adjacent lanes (lane & 3 = group m), and the
+// block's scale.  Only lanes with `store` write.
+__device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint4 *rec, float *scale, uint32_t m, bool store) {
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[i]));
+#pragma unroll
+  for (int off = 1; off < 4; off <<= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, off, 64));
+  if (!store) return;
+  const BlockScale bs = make_block_scale_q8(amax);
+  v8h q;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) q[i] = (_Float16)quantize_elem_q8(v[i], bs.inv);
+  *rec = __builtin_bit_cast(uint4, q);
+  if (m == 0) *scale = bs.s;
+}
+
+// Eight elements of block b, k-group m of the f32 vector x, in kgroup_elem order.
+template <int FMT>
+__device__ __forceinline__ void load_group(const float *x, uint32_t b, uint32_t m, float (&v)[8]) {
+  const float *xb = x + (size_t)b * 32;
+  const float4 lo = *reinterpret_cast<const float4 *>(xb + kgroup_elem<FMT>(m, 0));
+  const float4 hi = *reinterpret_cast<const float4 *>(xb + kgroup_elem<FMT>(m, 0) + (FMT == FMT_Q4_0 ? 16 : 4));
+  const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t e = kgroup_elem<FMT>(0, i);
+    v[i] = f[e >= 16 ? e - 12 : e];
+  }
+}
+
+__device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }  // -126..127
+
+// kF16Pair records (per block the four k-groups' high parts, then their low
+// parts) and scale of one f32 vector of `blocks` blocks, by the whole
+// workgroup; a non-finite vector gets a NaN scale.  Two passes over x: the
+// second reads caches.
+template <int FMT>
+__device__ __forceinline__ void quant_vector(const float *x, uint32_t blocks, uint4 *rec, float *scale) {
+  __shared__ float red[16];
+  const uint32_t groups = blocks * 4;
+  float amax = 0.f;
+  int finite = 1;
+  for (uint32_t g = threadIdx.x; g < groups; g += blockDim.x) {
     float v[8];
-    if (valid) {
-      const float4 a = *reinterpret_cast<const float4 *>(p.x + (size_t)tb * 32 + 8 * m);
-      const float4 b = *reinterpret_cast<const float4 *>(p.x + (size_t)tb * 32 + 8 * m + 4);
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-      v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
+    load_group<FMT>(x, g / 4, g % 4, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      amax = __builtin_fmaxf(amax, __builtin_fabsf(v[i]));
+      finite &= __builtin_isfinite(v[i]) ? 1 : 0;
+    }
+  }
+  if (!finite) amax = INFINITY;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, off, 64));
+  if (lane_id() == 0) red[threadIdx.x / 64] = amax;
+  __syncthreads();
+  for (uint32_t w = 0; w < blockDim.x / 64; ++w) amax = __builtin_fmaxf(amax, red[w]);
+  const bool ok = __builtin_isfinite(amax);
+  const int e = max((int)(__float_as_uint(amax) >> 23) - 127, -112);  // amax >= 0
+  const float inv = ok ? pow2f(14 - e) : 0.f;
+  if (threadIdx.x == 0) *scale = ok ? pow2f(e - 14) : __builtin_nanf("");
+  for (uint32_t g = threadIdx.x; g < groups; g += blockDim.x) {
+    float v[8];
+    load_group<FMT>(x, g / 4, g % 4, v);
+    if (!ok) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = 0.f;
     }
-    quant_group(v, p.xg + ((size_t)tb * 4 + m) * kGRec, valid, p.q8act != 0);
+    v8h hi, lo;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float y = v[i] * inv;
+      hi[i] = (_Float16)y;
+      lo[i] = (_Float16)(y - (float)hi[i]);
+    }
+    uint4 *r = rec + (size_t)(g / 4) * 8 + g % 4;
+    r[0] = __builtin_bit_cast(uint4, hi);
+    r[4] = __builtin_bit_cast(uint4, lo);
+  }
+}
+
+// Block 0: group the routed pairs by expert.  Other blocks: x's records.
+template <int FMT, int MODE>
+__global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
+  if (blockIdx.x > 0) {
+    if constexpr (MODE == kF16Pair) {  // one token per workgroup
+      const uint32_t t = blockIdx.x - 1;
+      quant_vector<FMT>(p.x + (size_t)t * p.d_model, p.xblocks, reinterpret_cast<uint4 *>(p.xg) + (size_t)t * p.xblocks * 8,
+                        p.xs + t);
+    } else {
+      const uint32_t g = (blockIdx.x - 1) * blockDim.x + threadIdx.x;  // (token, block, group)
+      const uint32_t total = p.n_tok * p.xblocks * 4;
+      // whole quads stay together for the shuffles; quads past the end idle
+      const bool valid = g < total;
+      const uint32_t tb = g / 4, m = g % 4;
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if constexpr (MODE == kQ8Act) {
+        if (valid) load_group<FMT>(p.x, tb, m, v);
+        quant_group_q8(v, reinterpret_cast<uint4 *>(p.xg) + (size_t)tb * 4 + m, p.xs + tb, m, valid);
+      } else {
+        if (valid) load_group<FMT_Q8_0>(p.x, tb, m, v);  // eight consecutive elements
+        quant_group(v, p.xg + ((size_t)tb * 4 + m) * kGRec, valid, p.q8act != 0);
+      }
+    }
     return;
   }
 
+  constexpr uint32_t kTile = MODE == kDigits ? kGTok : kBigTok;
   extern __shared__ uint32_t sh[];
   uint32_t *cnt = sh;                   // [table_len] pairs per expert, then offsets
   uint32_t *tcnt = sh + p.table_len;    // [table_len] tiles per expert, then offsets
@@ -199,7 +344,7 @@ __global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
   for (uint32_t e = e0; e < e1; ++e) {
     const uint32_t c = cnt[e];
     sp += c;
-    st += (c + kGTok - 1) / kGTok;
+    st += (c + kTile - 1) / kTile;
   }
   // Inclusive scan of (sp, st) over the block: within each wave by lane
   // shuffles, then over the wave totals (two barriers in all).
@@ -230,14 +375,16 @@ __global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
   uint32_t op = ip - sp, ot = it - st;
   for (uint32_t e = e0; e < e1; ++e) {
     const uint32_t c = cnt[e];
-    const uint32_t nt = (c + kGTok - 1) / kGTok;
+    const uint32_t nt = (c + kTile - 1) / kTile;
     cnt[e] = op;
     tcnt[e] = ot;
+    // 64-pair tiles of equal size, in whole groups of 16 pairs
+    const uint32_t size = kTile == kGTok || nt < 2 ? kTile : ((c + nt - 1) / nt + 15) / 16 * 16;
     for (uint32_t j = 0; j < nt; ++j) {
       GroupTile t;
       t.blob = reinterpret_cast<const uint8_t *>(p.table[e]);
-      t.start = op + j * kGTok;
-      t.count = min(kGTok, c - j * kGTok);
+      t.start = op + j * size;
+      t.count = min(size, c - j * size);
       p.tiles[ot + j] = t;
     }
     op += c;
@@ -249,12 +396,14 @@ __global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
     if (pos[q] != 0xffffffffu) p.plist[cnt[pos[q] >> 16] + (pos[q] & 0xffffu)] = q;
 }
 
+// ---- gproj: int8 MFMA, tiles of 16 pairs ----------------------------------
+
 // Stage one (16 RT)-row x (32 / RT)-block slab of weights into LDS: one
 // two-block chunk per thread, loaded with raw buffer loads into a register
 // buffer (a chunk past the row's end reads zeros) and stored as int8 rows
 // plus f32 scales.
 template <int FMT, int RT>
-struct Stager {
+struct DigitStager {
   using Geo = GGeom<RT>;
   using T = FmtTraits<FMT>;
   static constexpr int kDw = T::kChunkDwords;
@@ -284,7 +433,7 @@ struct Stager {
   // instead of merging two versions of them after a branch.
   __device__ __forceinline__ void load(uint32_t s, uint32_t row_chunks, Buf &w) const {
     const bool ok = s * Geo::kStageChunks + schunk < row_chunks;
-    const uint32_t off = ok ? voff + s * Geo::kStageChunks * (uint32_t)T::kChunkBytes : kNoChunkG;
+    const uint32_t off = ok ? voff + s * Geo::kStageChunks * (uint32_t)T::kChunkBytes : kNoLoad;
 #pragma unroll
     for (int v = 0; v < kDw / 4; ++v) {
       const uint4 q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 16 * v, 0, 0));
@@ -345,7 +494,7 @@ struct Stager {
 template <int FMT, bool FUSED, int RT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGWavesPerEu))) void gproj_kernel(GroupedParams p) {
   using Geo = GGeom<RT>;
-  using SG = Stager<FMT, RT>;
+  using SG = DigitStager<FMT, RT>;
   constexpr uint32_t kRows = Geo::kRows, kSB = Geo::kStageBlocks, kStride = Geo::kRowStride, kSS = Geo::kScaleStride;
   constexpr int kWB = Geo::kWaveBlocks;
   // Two LDS slabs: stage s + 1 is stored into one while stage s is read
@@ -544,9 +693,443 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGWavesPerE
   }
 }
 
+// ---- gbig: tiles of up to 64 pairs, shared parts ---------------------------
+
+// f16 weights of one MFMA k-group from its raw bytes (exact integers).
+// Q4_0: qs dword -> q - 8 of bytes' low and high nibbles, in kgroup_elem
+// order: (1024 + n) - 1032, and (1024 + 16 n) / 16 - 72 for high nibbles.
+// NEG: the negated weights.
+template <bool NEG>
+__device__ __forceinline__ v8h unpack_q4(uint32_t w) {
+  const v2h c1 = {(_Float16)1032.0f, (_Float16)1032.0f};
+  const v2h c2 = {(_Float16)72.0f, (_Float16)72.0f};
+  const v2h r = {(_Float16)0.0625f, (_Float16)0.0625f};
+  const uint32_t w8 = w >> 8;
+  const v2h a = __builtin_bit_cast(v2h, (w & 0x000f000fu) | 0x64006400u);
+  const v2h b = __builtin_bit_cast(v2h, (w & 0x00f000f0u) | 0x64006400u);
+  const v2h c = __builtin_bit_cast(v2h, (w8 & 0x000f000fu) | 0x64006400u);
+  const v2h d = __builtin_bit_cast(v2h, (w8 & 0x00f000f0u) | 0x64006400u);
+  const v2h e = NEG ? c1 - a : a - c1, f = NEG ? c2 - b * r : b * r - c2;
+  const v2h g = NEG ? c1 - c : c - c1, h = NEG ? c2 - d * r : d * r - c2;
+  return v8h{e.x, e.y, f.x, f.y, g.x, g.y, h.x, h.y};
+}
+// Q8_0: eight consecutive int8: (1024 + (q + 128)) - 1152.
+template <bool NEG>
+__device__ __forceinline__ v8h unpack_q8(uint32_t lo, uint32_t hi) {
+  const v2h c = {(_Float16)1152.0f, (_Float16)1152.0f};
+  lo ^= 0x80808080u;
+  hi ^= 0x80808080u;
+  const v2h a = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u));
+  const v2h b = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u));
+  const v2h d = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u));
+  const v2h e = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u));
+  const v2h f = NEG ? c - a : a - c, g = NEG ? c - b : b - c, h = NEG ? c - d : d - c, i = NEG ? c - e : e - c;
+  return v8h{f.x, f.y, g.x, g.y, h.x, h.y, i.x, i.y};
+}
+
+// Asynchronous copy of 16 bytes per lane from a buffer (an offset past its
+// end reads zeros) to LDS at `lds` + 16 * lane.  The compiler does not see
+// it: the caller waits (wait_vm) before the barrier that publishes it.  M0
+// holds the LDS address; s_nop: wait states between a write of M0 or of a
+// resource word and its use.
+__device__ __forceinline__ void async_lds16(v4u rsrc, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds) : "memory");
+}
+// The same for 4 bytes per lane, to LDS at `lds` + 4 * lane.
+__device__ __forceinline__ void async_lds4(v4u rsrc, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds) : "memory");
+}
+// Wait until at most N of this wave's vector memory operations are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// The same and this wave's LDS reads, then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void wait_vm_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// A workgroup's item: a token tile and a row tile (with a K part folded in by
+// the caller).  Items are ordered expert, token tile, row tile, and runs of
+// them go to one XCD: its workgroups then share one tile's inputs in their L2
+// (Mixtral prefill, 2048 tokens: 3.45 ms, 3.73 with the token tiles of a row
+// tile together).
+struct GItem {
+  const uint8_t *blob;
+  uint32_t start, count, rt;
+};
+__device__ __forceinline__ bool group_item(const GroupedParams &p, uint32_t row_tiles, GItem *it) {
+  const uint32_t total = *p.n_tiles * row_tiles;
+  const uint32_t x = blockIdx.x % 8, q = blockIdx.x / 8;
+  const uint32_t run = max(1u, min(total / 64, kGMaxRun));
+  const uint32_t item = ((q / run) * 8 + x) * run + q % run;
+  if (item >= total) return false;
+  const GroupTile gt = p.tiles[item / row_tiles];
+  it->blob = gt.blob;
+  it->rt = item % row_tiles;
+  it->start = gt.start;
+  it->count = gt.count;
+  return true;
+}
+
+// kBigRows weight rows by NG groups of 32 pairs on v_mfma_f32_32x32x16_f16.
+// The waves split the rows (64 each) and share every block of inputs, so
+// inputs and weights both go through LDS, copied asynchronously four blocks
+// and a stage ahead: no load returns to registers inside the loop, so none
+// waits behind another (a wave's loads return in order).  Lane l of a 32 x 32
+// product holds weight row l % 32 and pairs 8 (i / 4) + 4 (l / 32) + i % 4.
+//
+// Bound: matrix unit and vector issue slots at the clock the power limit
+// leaves (Mixtral Q4_0, 4096 pairs: 1.8 GHz, 49% and 59% of cycles busy; the
+// two f16 products alone take 1.4 ms of the gate/up launch's 2.15 at the
+// rate the unit sustains on such data).  One product of a wave's own has to
+// saturate the unit while its other wave works on sums, which 32 x 32 tiles
+// do and 16 x 16 tiles do not.  Mixtral Q4_0 top-2, 2048 tokens, against the
+// int8 kernel: gate/up 4.49 -> 2.15 ms, down 2.16 -> 1.1 ms; 333 tokens under
+// MER_MOE_QMM 0.84 -> 0.46 and 0.42 -> 0.24 ms (its products are half as many,
+// its sums carry a scale per pair as well: vector issue).
+constexpr uint32_t kBigRows = 256;
+constexpr uint32_t kBigGran = 5;                          // 16-byte granules per staged row segment
+constexpr uint32_t kBigStride = 16 * kBigGran;
+constexpr uint32_t kBigSlab = kBigRows * kBigStride;
+constexpr uint32_t kXSlots = 5;
+constexpr uint32_t kX0 = 2 * kBigSlab;                    // LDS offset of the input slots
+// LDS bytes of a block of 64 pairs' inputs: records, or records and scales
+template <int MODE> constexpr uint32_t kXSlot = MODE == kF16Pair ? 64 * 128 : 64 * 64 + 4 * 256;
+
+template <int FMT, int MODE, bool FUSED, int NG>
+struct GBig {
+  static constexpr int kParts = MODE == kF16Pair ? 2 : 1;  // f16 parts of an input
+  static constexpr uint32_t kBB = FmtTraits<FMT>::kBlockBytes;
+  static constexpr int kSB = FMT == FMT_Q4_0 ? 4 : 2;      // blocks per stage: 72 or 68 of 80 bytes
+  static constexpr int kNW = (int)(kBigRows * kBigGran / 256);  // weight copies per wave and stage
+  static constexpr uint32_t kFlush = 16 / kSB;             // stages per partial sum
+  static constexpr int kXCopies = 2 * NG * kParts / 4 ? 2 * NG * kParts / 4 : 1;
+  // input copies per wave and block: records, and under kQ8Act scales
+  static constexpr int kNX = kXCopies + (MODE == kQ8Act ? 1 : 0);
+  static constexpr int kQW = FMT == FMT_Q4_0 ? 3 : 5;      // LDS words a lane reads per row and block
+  static_assert(kXSlots == 5, "inputs are copied four blocks ahead");
+  static_assert(kBigRows * kBigGran % 256 == 0, "whole copies");
+
+  static __device__ __forceinline__ void run(const GroupedParams &p, const uint8_t *blob, uint32_t start, uint32_t count,
+                                             uint32_t rt, uint32_t part, uint8_t *lds) {
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(tid / 64u);
+    const uint32_t rows = FUSED ? p.d_ff : p.d_model;
+    const uint32_t row_blocks = FUSED ? p.xblocks : p.hblocks;
+    // the blocks of this K part (whole stages; parts divide gate/up never)
+    const uint32_t b0 = FUSED ? 0u : part * p.part_blocks;
+    const uint32_t kblocks = FUSED ? row_blocks : min(p.part_blocks, row_blocks - b0);
+    const uint32_t n_stages = (kblocks + kSB - 1) / kSB;
+    constexpr uint32_t kOwnRows = FUSED ? kBigRows / 2 : kBigRows;
+    const uint32_t row0 = rt * kOwnRows;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+
+    // Weights: staged rows are 128 gate rows then the same 128 up rows
+    // (FUSED), or 256 down rows, kBigGran granules each.  Rows past the
+    // matrix read zeros; the buffer ends with the projection, so granules
+    // that overhang its last row read zeros too.
+    const uint64_t wb = reinterpret_cast<uint64_t>(blob) + (FUSED ? 0 : 2 * p.proj_bytes);
+    const v4u wr = {(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)wb),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(wb >> 32)),
+                    (uint32_t)((FUSED ? 2 : 1) * p.proj_bytes), 0x00020000u};
+    uint32_t woff[kNW];
+#pragma unroll
+    for (int j = 0; j < kNW; ++j) {
+      const uint32_t g = tid + 256u * j;
+      const uint32_t r = g / kBigGran, gi = g % kBigGran;
+      const uint32_t own = FUSED ? r % kOwnRows : r;
+      const bool ok = row0 + own < rows;
+      woff[j] = ok ? (FUSED && r >= kOwnRows ? (uint32_t)p.proj_bytes : 0u) + (row0 + own) * (row_blocks * kBB) + b0 * kBB + 16u * gi : kNoLoad;
+    }
+    uint32_t w_issued = 0;
+    auto issue_w = [&]() {
+      const uint32_t none = w_issued < n_stages ? 0u : kNoLoad;
+#pragma unroll
+      for (int j = 0; j < kNW; ++j) {
+        async_lds16(wr, woff[j] | none, lds0 + (w_issued & 1u) * kBigSlab + wave * 1024u + 4096u * j);
+        woff[j] += kSB * kBB;
+      }
+      ++w_issued;
+    };
+    // Inputs: copy i takes part i % kParts of the 16 vectors i / kParts; lane l
+    // copies k-group l / 16 of vector l % 16 (64 contiguous bytes per
+    // vector).  Wave w makes copies w, w + 4 (of 2 NG kParts; where there are
+    // fewer than four, waves repeat them).
+    const uint32_t vec_bytes = row_blocks * 64u * kParts;
+    const uint32_t n_vec = FUSED ? p.n_tok : p.n_pairs;
+    const uint64_t xbase = reinterpret_cast<uint64_t>(FUSED ? p.xg : p.hg);
+    const v4u xr = {(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)xbase),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(xbase >> 32)), n_vec * vec_bytes, 0x00020000u};
+    uint32_t xoff[kXCopies], soff = kNoLoad;
+    v4u sr = xr;
+    if constexpr (MODE == kQ8Act) {
+      const uint64_t sbase = reinterpret_cast<uint64_t>(FUSED ? p.xs : p.hs);
+      sr = v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)sbase),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(sbase >> 32)), n_vec * row_blocks * 4u, 0x00020000u};
+    }
+#pragma unroll
+    for (int j = 0; j < kXCopies; ++j) {
+      const uint32_t i = (wave + 4u * j) % (2 * NG * kParts);
+      const uint32_t n = 16 * (i / kParts) + lane % 16;
+      const uint32_t pair = n < count ? p.plist[start + n] : 0u;
+      // a column without a pair reads zeros
+      xoff[j] = n < count ? (FUSED ? pair / p.top_k : pair) * vec_bytes + b0 * 64u * kParts + 64u * (i % kParts) + 16u * (lane / 16) : kNoLoad;
+      if (MODE == kQ8Act && n < count) soff = ((FUSED ? pair / p.top_k : pair) * row_blocks + b0) * 4u;
+    }
+    uint32_t x_issued = 0, x_slot = 0;
+    auto issue_x = [&]() {
+      const uint32_t none = x_issued < kblocks ? 0u : kNoLoad;
+#pragma unroll
+      for (int j = 0; j < kXCopies; ++j) {
+        async_lds16(xr, xoff[j] | none, lds0 + kX0 + x_slot * kXSlot<MODE> + (wave + 4u * j) % (2 * NG * kParts) * 1024u);
+        xoff[j] += 64u * kParts;
+      }
+      if constexpr (MODE == kQ8Act) {  // the scales of the copy's 16 vectors, four times over
+        async_lds4(sr, soff | none, lds0 + kX0 + x_slot * kXSlot<MODE> + 4096u + wave % (2 * NG) * 256u);
+        soff += 4u;
+      }
+      ++x_issued;
+      x_slot = x_slot + 1 == kXSlots ? 0u : x_slot + 1;
+    };
+
+    // Sums over kFlush stages in acc, of those in tot: an f32 rounding error
+    // then grows with 16 + K / 512 terms instead of K / 32.
+    v16f acc[2][NG], tot[2][NG];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[a][g][i] = tot[a][g][i] = 0.f;
+
+    v8h wv[2][2];
+    float dw[2];
+    struct Raw {
+      uint32_t q[kQW];
+      _Float16 d;
+    };
+    // the wave's two row tiles: 32 gate rows and the same up rows, or 64 down rows
+    const uint32_t trow = (FUSED ? 32 * wave : 64 * wave) + lane % 32;
+    constexpr uint32_t kTileStep = (FUSED ? kOwnRows : 32) * kBigStride;
+    auto fetch = [&](const uint8_t *sl, uint32_t at, int a) {
+      const uint8_t *lr = sl + trow * kBigStride + a * kTileStep;
+      const uint32_t *q =
+          reinterpret_cast<const uint32_t *>(lr + ((at + 2 + (FMT == FMT_Q4_0 ? 8 : 16) * (lane / 32)) & ~3u));
+      Raw r;
+#pragma unroll
+      for (int i = 0; i < kQW; ++i) r.q[i] = q[i];
+      r.d = *reinterpret_cast<const _Float16 *>(lr + at);
+      return r;
+    };
+    auto unpack = [&](auto neg, const Raw &r, uint32_t at, uint32_t live, int a) {
+      constexpr bool kNeg = decltype(neg)::value;
+      const uint32_t sh = (at & 2u) ? 0u : 16u;  // qs start 2 bytes past a dword in even blocks
+      uint32_t q[kQW - 1];
+#pragma unroll
+      for (int i = 0; i + 1 < kQW; ++i) q[i] = __builtin_amdgcn_alignbit(r.q[i + 1], r.q[i], sh);
+      if constexpr (FMT == FMT_Q4_0) {
+        wv[a][0] = unpack_q4<kNeg>(q[0]);
+        wv[a][1] = unpack_q4<kNeg>(q[1]);
+      } else {
+        wv[a][0] = unpack_q8<kNeg>(q[0], q[1]);
+        wv[a][1] = unpack_q8<kNeg>(q[2], q[3]);
+      }
+      const float d = (float)r.d;
+      dw[a] = __uint_as_float(__float_as_uint(kNeg ? -d : d) & live);
+    };
+    // input operands of group g: [k step][high, low part]; lane l takes
+    // vector l % 32, k-group 2 (l / 32) + k (as the weights' words do)
+    v8h x[NG][2][kParts];
+    float f[16];  // kQ8Act: the scales of the lane's output pairs of one group
+    const uint32_t xlane = ((lane % 32) / 16) * (1024u * kParts) + (lane / 32) * 512u + (lane % 16) * 16u;
+    auto read_x = [&](const uint8_t *slot, int g) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int part = 0; part < kParts; ++part)
+          x[g][k][part] = *reinterpret_cast<const v8h *>(slot + xlane + g * (2048u * kParts) + part * 1024u + k * 256u);
+    };
+    auto read_f = [&](const uint8_t *slot, int g) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 v = *reinterpret_cast<const float4 *>(slot + 4096u + (2 * g + q / 2) * 256u + (8 * (q % 2) + 4 * (lane / 32)) * 4u);
+        f[4 * q] = v.x;
+        f[4 * q + 1] = v.y;
+        f[4 * q + 2] = v.z;
+        f[4 * q + 3] = v.w;
+      }
+    };
+
+    // Start: the copies of stages 0 and 1 and of blocks 0..3, in the loop's order.
+    issue_w();
+    issue_x();
+    issue_x();
+    issue_x();
+    issue_w();
+    issue_x();
+    wait_vm_barrier<3 * kNX + kNW>();
+    {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) unpack(std::false_type{}, fetch(lds, 0u, a), 0u, 0xffffffffu, a);
+#pragma unroll
+      for (int g = 0; g < NG; ++g) read_x(lds + kX0, g);
+    }
+    // Block b: at its barrier the inputs of block b + 1 (and, before the
+    // stage's last block, the next stage's weights) are complete, and the
+    // inputs of block b are in every wave's registers, so the slot of block
+    // b - 1 takes block b + 4.
+    uint32_t xs = 0;
+    auto stage = [&](uint32_t s) {
+      const uint8_t *cur = lds + (s & 1u) * kBigSlab, *nxt = lds + ((s & 1u) ^ 1u) * kBigSlab;
+      auto block = [&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        // Copies started after those of block b + 1 (at block b - 3): the
+        // inputs of two blocks, and weights if one of these was a stage's
+        // last block.  A stage's last block needs the next stage's weights
+        // too, started kSB blocks before.
+        constexpr bool kEnd = j == kSB - 1;
+        constexpr int kYoungX = 2 * kNX + ((j + kSB - 1) % kSB == kSB - 1 || (j + 2 * kSB - 2) % kSB == kSB - 1 ? kNW : 0);
+        constexpr int kYoungW = kSB * kNX;
+        wait_vm_barrier<(kEnd && kYoungW < kYoungX ? kYoungW : kYoungX)>();
+        // the slab's last block is in registers: the slab takes stage s + 2
+        if constexpr (kEnd) issue_w();
+        issue_x();
+        const uint8_t *xc = lds + kX0 + xs * kXSlot<MODE>;
+        xs = xs + 1 == kXSlots ? 0u : xs + 1;
+        const uint8_t *xn = lds + kX0 + xs * kXSlot<MODE>;
+        constexpr uint32_t nat = kEnd ? 0u : (uint32_t)(j + 1) * kBB;
+        const uint8_t *nsl = kEnd ? nxt : cur;
+        constexpr std::bool_constant<!kEnd && (j + 1) % 2 == 1> next_odd{};
+        const uint32_t live = s * kSB + j + 1 < kblocks ? 0xffffffffu : 0u;
+        v16f t[2];
+        Raw raw[2];
+        auto finish = [&](int g, int a) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[a][g][i] = __builtin_fmaf(t[a][i], MODE == kQ8Act ? dw[a] * f[i] : dw[a], acc[a][g][i]);
+          if (g == NG - 1) unpack(next_odd, raw[a], nat, live, a);
+        };
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int a = 0; a < 2; ++a) {
+            if (g == NG - 1) raw[a] = fetch(nsl, nat, a);
+            v16f z;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) z[i] = 0.f;
+            v16f r = z;
+#pragma unroll
+            for (int part = kParts - 1; part >= 0; --part)
+#pragma unroll
+              for (int k = 0; k < 2; ++k) r = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[g][k][part], wv[a][k], r, 0, 0, 0);
+            t[a] = r;
+            if (g > 0 || a > 0) {
+              finish(a ? g : g - 1, a ^ 1);
+              // products and sums in turn: a product occupies the matrix unit
+              // long enough for sums of the tile before it to issue
+              __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+              for (int i = 0; i < 2 * kParts; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (g == NG - 1 && a == 1) __builtin_amdgcn_sched_group_barrier(0x002, MODE == kQ8Act ? 28 : 10, 0);
+                else __builtin_amdgcn_sched_group_barrier(0x002, MODE == kQ8Act ? 16 : 4, 0);
+              }
+            }
+            if (MODE == kQ8Act && a == 0) read_f(xc, g);  // (after the sums that use the last group's)
+            __builtin_amdgcn_sched_barrier(0);
+            if (a == 1) read_x(xn, g);
+          }
+        finish(NG - 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      block(std::integral_constant<int, 0>{});
+      block(std::integral_constant<int, 1>{});
+      if constexpr (kSB == 4) {
+        block(std::integral_constant<int, 2>{});
+        block(std::integral_constant<int, 3>{});
+      }
+    };
+    for (uint32_t s0 = 0; s0 < n_stages; s0 += kFlush) {
+      for (uint32_t s = s0; s < min(n_stages, s0 + kFlush); ++s) stage(s);
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            tot[a][g][i] += acc[a][g][i];
+            acc[a][g][i] = 0.f;
+          }
+    }
+    wait_vm<0>();
+    __syncthreads();  // nothing writes LDS any more
+
+    // each pair's output row and factor, read back by every lane's rows
+    uint64_t *prow = reinterpret_cast<uint64_t *>(lds);
+    float *pscale = reinterpret_cast<float *>(lds + 64 * 8);
+    if (tid < 32 * NG && tid < count) {
+      const uint32_t pr = p.plist[start + tid];
+      prow[tid] = reinterpret_cast<uint64_t>(FUSED ? p.h32 + (size_t)pr * p.d_ff : p.partial + ((size_t)part * p.n_pairs + pr) * p.d_model);
+      const float sc = MODE == kQ8Act ? 1.0f : FUSED ? p.xs[pr / p.top_k] : p.hs[pr];  // the vector's scale
+      pscale[tid] = !FUSED && p.weights ? sc * p.weights[pr] : sc;
+    }
+    __syncthreads();
+    const uint32_t r = row0 + trow;
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t n = 32 * g + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
+        if (n >= count) continue;
+        float *out = reinterpret_cast<float *>(prow[n]);
+        const float sc = pscale[n];
+        if constexpr (FUSED) {
+          if (r < rows) out[r] = silu_mul(tot[0][g][i] * sc, tot[1][g][i] * sc, p.swiglu_limit);
+        } else {
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+            if (r + 32 * a < rows) out[r + 32 * a] = sc * tot[a][g][i];
+        }
+      }
+  }
+};
+
+template <int FMT, int MODE, bool FUSED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gbig_kernel(GroupedParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kX0 + kXSlots * kXSlot<MODE>];  // two workgroups per CU
+  const uint32_t parts = FUSED ? 1u : p.n_parts;
+  GItem it;
+  if (!group_item(p, ((FUSED ? 2 * p.d_ff : p.d_model) + kBigRows - 1) / kBigRows * parts, &it)) return;  // uniform
+  const uint32_t rt = it.rt / parts, part = it.rt % parts;
+  if (it.count > 32) GBig<FMT, MODE, FUSED, 2>::run(p, it.blob, it.start, it.count, rt, part, lds);
+  else GBig<FMT, MODE, FUSED, 1>::run(p, it.blob, it.start, it.count, rt, part, lds);
+}
+
+// The records of h for gbig's down projection, one workgroup per routed pair.
+template <int FMT, int MODE>
+__global__ __launch_bounds__(256) void hquant_kernel(GroupedParams p) {
+  const uint32_t pair = blockIdx.x;
+  if (!p.pair_ok[pair]) return;
+  const float *h = p.h32 + (size_t)pair * p.d_ff;
+  if constexpr (MODE == kF16Pair) {
+    quant_vector<FMT>(h, p.hblocks, reinterpret_cast<uint4 *>(p.hg) + (size_t)pair * p.hblocks * 8, p.hs + pair);
+  } else {
+    // whole quads of lanes per block; d_ff / 8 groups are a multiple of 8
+    for (uint32_t g = threadIdx.x; g < p.hblocks * 4; g += blockDim.x) {
+      const size_t b = (size_t)pair * p.hblocks + g / 4;
+      float v[8];
+      load_group<FMT>(h, g / 4, g % 4, v);
+      quant_group_q8(v, reinterpret_cast<uint4 *>(p.hg) + b * 4 + g % 4, p.hs + b, g % 4, true);
+    }
+  }
+}
+
 // out[t] = [x +] sum over the token's valid slots, in slot order, of the
 // pair partials (w_i y_i).  One thread per 4 output elements; the slots'
 // validity comes from the grouping kernel, so all loads are independent.
+// PARTS: the pairs' sums come in K parts.
+template <bool PARTS>
 __global__ __launch_bounds__(256) void gcombine_kernel(GroupedParams p) {
   const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t per_tok = p.d_model / 4;
@@ -565,6 +1148,16 @@ __global__ __launch_bounds__(256) void gcombine_kernel(GroupedParams p) {
     for (uint32_t j = 0; j < 8; ++j)
       v[j] = ok[j] ? *reinterpret_cast<const float4 *>(p.partial + (size_t)(t * p.top_k + k0 + j) * p.d_model + c)
                    : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t part = 1; PARTS && part < p.n_parts; ++part) {  // in order
+      float4 u[8];
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j)
+        u[j] = ok[j] ? *reinterpret_cast<const float4 *>(
+                           p.partial + ((size_t)part * p.n_pairs + t * p.top_k + k0 + j) * p.d_model + c)
+                     : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) v[j] = make_float4(v[j].x + u[j].x, v[j].y + u[j].y, v[j].z + u[j].z, v[j].w + u[j].w);
+    }
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j)
       if (ok[j]) {
@@ -589,14 +1182,22 @@ size_t grouped_group_lds_bytes(uint32_t table_len, uint32_t n_pairs) {
   return (size_t)(2 * table_len + n_pairs) * 4;
 }
 
-hipError_t launch_grouped_prep(const GroupedParams &p, hipStream_t st) {
+template <int FMT, int MODE>
+static hipError_t launch_gprep(const GroupedParams &p, hipStream_t st) {
   const uint32_t quads = p.n_tok * p.xblocks * 4;
-  const uint32_t gblocks = 1 + (quads + 1023) / 1024;
-  hipLaunchKernelGGL(group_kernel, dim3(gblocks), dim3(1024), grouped_group_lds_bytes(p.table_len, p.n_pairs), st, p);
+  const uint32_t gblocks = 1 + (MODE == kF16Pair ? p.n_tok : (quads + 1023) / 1024);
+  hipLaunchKernelGGL((group_kernel<FMT, MODE>), dim3(gblocks), dim3(1024), grouped_group_lds_bytes(p.table_len, p.n_pairs), st,
+                     p);
   return hipGetLastError();
 }
 
-hipError_t launch_grouped_proj(int fmt, bool fused, const GroupedParams &p, uint32_t max_tiles, hipStream_t st) {
+hipError_t launch_grouped_prep(int fmt, const GroupedParams &p, hipStream_t st) {
+  if (p.mode == kDigits) return launch_gprep<FMT_Q8_0, kDigits>(p, st);  // one layout for both formats
+  if (p.mode == kQ8Act) return launch_gprep<FMT_Q4_0, kQ8Act>(p, st);
+  return fmt == FMT_Q4_0 ? launch_gprep<FMT_Q4_0, kF16Pair>(p, st) : launch_gprep<FMT_Q8_0, kF16Pair>(p, st);
+}
+
+static hipError_t launch_gproj(int fmt, bool fused, const GroupedParams &p, uint32_t max_tiles, hipStream_t st) {
   // Down runs 128-row workgroups (RT = 8) wherever d_model divides by 128.
   // Gate/up does so (64 gate + 64 up rows) only from 2048 routed pairs on:
   // with fewer its launch fills too few rounds of the resident workgroup
@@ -623,9 +1224,36 @@ hipError_t launch_grouped_proj(int fmt, bool fused, const GroupedParams &p, uint
   return hipGetLastError();
 }
 
+template <int FMT, int MODE, bool FUSED>
+static hipError_t launch_gbig(const GroupedParams &p, uint32_t max_tiles, hipStream_t st) {
+  const uint32_t row_tiles = ((FUSED ? 2 * p.d_ff : p.d_model) + kBigRows - 1) / kBigRows * (FUSED ? 1u : p.n_parts);
+  // whole runs of items on each XCD: up to one run per XCD past the items
+  const dim3 grid((max_tiles * row_tiles + 7) / 8 * 8 + 8 * kGMaxRun);
+  hipLaunchKernelGGL((gbig_kernel<FMT, MODE, FUSED>), grid, dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+template <int FMT, int MODE>
+static hipError_t launch_gbig_mode(bool fused, const GroupedParams &p, uint32_t max_tiles, hipStream_t st) {
+  if (!fused) return launch_gbig<FMT, MODE, false>(p, max_tiles, st);
+  const hipError_t e = launch_gbig<FMT, MODE, true>(p, max_tiles, st);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((hquant_kernel<FMT, MODE>), dim3(p.n_pairs), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_grouped_proj(int fmt, bool fused, const GroupedParams &p, uint32_t max_tiles, hipStream_t st) {
+  if (p.mode == kDigits) return launch_gproj(fmt, fused, p, max_tiles, st);
+  if (p.mode == kQ8Act) return launch_gbig_mode<FMT_Q4_0, kQ8Act>(fused, p, max_tiles, st);
+  return fmt == FMT_Q4_0 ? launch_gbig_mode<FMT_Q4_0, kF16Pair>(fused, p, max_tiles, st)
+                         : launch_gbig_mode<FMT_Q8_0, kF16Pair>(fused, p, max_tiles, st);
+}
+
 hipError_t launch_grouped_combine(const GroupedParams &p, hipStream_t st) {
   const uint32_t cq = p.n_tok * (p.d_model / 4);
-  hipLaunchKernelGGL(gcombine_kernel, dim3((cq + 255) / 256), dim3(256), 0, st, p);
+  const dim3 grid((cq + 255) / 256);
+  if (p.n_parts > 1) hipLaunchKernelGGL(gcombine_kernel<true>, grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(gcombine_kernel<false>, grid, dim3(256), 0, st, p);
   return hipGetLastError();
 }
 

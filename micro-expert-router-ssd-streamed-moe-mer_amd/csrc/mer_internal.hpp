@@ -158,10 +158,13 @@ struct DecodeParams {
 constexpr uint32_t kMaxGroupedExperts = 4096;  // table entries the grouping kernel counts in LDS
 constexpr uint32_t kMaxGroupedPairs = 4096;    // routed (token, slot) pairs per call
 
+// Input formats of the projection kernels (mer_grouped.hip).
+enum GroupMode : uint32_t { kGroupDigits = 0, kGroupQ8Act = 1, kGroupF16Pair = 2 };
+
 struct GroupTile {
   const uint8_t *blob;  // the expert's blob
   uint32_t start;       // first pair of the tile in plist
-  uint32_t count;       // pairs in the tile (1..16)
+  uint32_t count;       // pairs in the tile: 1..16 (kGroupDigits) or 1..64
 };
 
 struct GroupedParams {
@@ -178,18 +181,22 @@ struct GroupedParams {
   float swiglu_limit;        // gate clamp before SiLU (+inf = none)
   size_t proj_bytes;
   // scratch
-  uint32_t *xg;              // x digit records [n_tok][xblocks][4 k-groups][8 dwords]
-  uint32_t *hg;              // h digit records [n_pairs][hblocks][4][8 dwords]
-  float *partial;            // w_i y_i [n_pairs][d_model]
+  uint32_t *xg;              // x records [n_tok][xblocks][4 k-groups], 8 dwords each (4 under kGroupQ8Act)
+  uint32_t *hg;              // h records [n_pairs][hblocks][4]
+  float *partial;            // w_i y_i [n_parts][n_pairs][d_model]
   uint32_t *plist;           // pairs grouped by expert [n_pairs]
   uint32_t *pair_ok;         // [n_pairs] 1 = routed to a resident expert with a nonzero weight
   GroupTile *tiles;          // [max tiles]
   uint32_t *n_tiles;         // tiles emitted by the grouping kernel
   uint32_t *status;
+  uint32_t mode;             // kGroupDigits, kGroupQ8Act or kGroupF16Pair
+  uint32_t n_parts, part_blocks;  // K parts of the down projection, blocks of each
+  float *xs, *hs;            // f16 modes: the scales of the records, per vector or (kGroupQ8Act) per block
+  float *h32;                // f16 modes: f32 h [n_pairs][d_ff]
 };
 
 size_t grouped_group_lds_bytes(uint32_t table_len, uint32_t n_pairs);
-hipError_t launch_grouped_prep(const GroupedParams &p, hipStream_t st);
+hipError_t launch_grouped_prep(int fmt, const GroupedParams &p, hipStream_t st);
 hipError_t launch_grouped_proj(int fmt, bool fused, const GroupedParams &p, uint32_t max_tiles, hipStream_t st);
 hipError_t launch_grouped_combine(const GroupedParams &p, hipStream_t st);
 

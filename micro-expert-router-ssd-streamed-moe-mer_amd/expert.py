@@ -258,7 +258,7 @@ def expert_matmul(dtype: WeightDtype, d_model: int, d_ff: int, table: torch.Tens
 def moe_grouped(dtype: WeightDtype, d_model: int, d_ff: int, table: torch.Tensor, expert_ids: torch.Tensor,
                 weights: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None = None, *,
                 residual: bool = False, accumulate: bool = False, qmm: bool = False) -> torch.Tensor:
-    """moe_forward for a multi-token batch on the grouped int8-MFMA path:
+    """moe_forward for a multi-token batch on the grouped MFMA path:
     pairs grouped by expert on the device, each expert's weights read once
     for all of its tokens (the batched routed_expert_matmul_batch_q4,
     backend/mod.rs:4401-4418).  Same arguments and combine as moe_forward;
