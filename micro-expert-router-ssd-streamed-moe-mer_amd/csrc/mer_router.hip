@@ -7,7 +7,11 @@
 //               router_logits_kernel: one wave per (expert, group of 4
 //               tokens), so the gate matrix streams through every CU
 //               with many loads in flight (one token reads all of W);
-//   the rest, one 256-thread workgroup per token (router_kernel):
+//               router_logits_mfma_kernel: 32 tokens x 32 experts per
+//               workgroup, for large batches;
+//   the rest, one wave per token (router_kernel; its top-k in registers and
+//   the weights of all slots at once: 11.5 -> 7.6 us for 2048 tokens, top-8 of
+//   128):
 //   scores    = softmax(logits) (transformer.rs:2807, non-finite rows fall
 //               back to uniform) or sigmoid (gating.rs:271-279)
 //   selection = scores + correction_bias          (bias optional)
@@ -28,6 +32,11 @@ namespace {
 constexpr int kRouterThreads = 256;
 constexpr int kRouterWaves = kRouterThreads / 64;
 constexpr uint32_t kRouterTokGroup = 4;  // tokens per logits wave
+constexpr uint32_t kRouterTile = 32;      // tokens and experts per workgroup of the MFMA kernel
+constexpr int kRouterMWaves = 8;           // its waves
+constexpr uint32_t kRouterStage = 16 * kRouterMWaves;  // its k-indices per stage
+constexpr uint32_t kRouterStride = kRouterStage + 4;   // LDS row, padded to spread banks
+typedef float v4f __attribute__((ext_vector_type(4)));
 // The per-token selection runs as one wave: its reductions are shuffles and
 // its barriers cost no waiting on other waves.
 constexpr int kSelThreads = 64;
@@ -132,18 +141,132 @@ __global__ __launch_bounds__(kRouterThreads) void router_logits_kernel(RouterPar
   }
 }
 
+// The same for many tokens: 32 tokens by 32 experts per workgroup on
+// v_mfma_f32_16x16x4_f32, so each element of x and W is loaded once per 32
+// logits instead of once per logit or per four.  Stages of 128 k-indices go
+// through LDS, read whole rows at a time: rows of a power-of-two length start
+// in one L2 channel and one L1 set, so 16 rows per load instruction (straight
+// from the operand layout) ran at a third of the rate; for the same reason
+// each workgroup starts at another stage.  Wave w takes the stage's run w of
+// 16 k-indices; lane l holds four consecutive elements of row l % 16
+// (k-indices 4 (l / 16) .. + 3 of the run), one for each of four products,
+// which is the same permutation of k on both sides.  Sums are kept short, as
+// they are in the kernel above (32 terms per lane): 16 products, eight of
+// those, the rest, then the waves.  Rows and k past the ends are 0.
+// ALIGNED: d_model % 4 == 0, so no 16 bytes hold two rows' elements.
+template <bool ALIGNED>
+__global__ __launch_bounds__(64 * kRouterMWaves) void router_logits_mfma_kernel(RouterParams p) {
+  __shared__ __attribute__((aligned(16))) float lds[2][2 * kRouterTile][kRouterStride];
+  // the workgroups of one token tile run on one XCD, whose L2 keeps its x
+  const uint32_t n_eg = (p.n_experts + kRouterTile - 1) / kRouterTile;
+  const uint32_t q = blockIdx.x / 8;
+  const uint32_t t0 = ((q / n_eg) * 8 + blockIdx.x % 8) * kRouterTile, e0 = (q % n_eg) * kRouterTile;
+  if (t0 >= p.n_tokens) return;  // the whole workgroup
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t row = lane % 16, kg = lane / 16;
+  // staging: thread t copies 16 bytes (column t % 32) of rows t / 32 + 16 j;
+  // rows 0..31 are tokens (j < 2), 32..63 experts
+  const uint32_t nt = min(kRouterTile, p.n_tokens - t0), ne = min(kRouterTile, p.n_experts - e0);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(p.x + (size_t)t0 * p.d_model), 0, nt * p.d_model * 4u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(p.gate + (size_t)e0 * p.d_model), 0, ne * p.d_model * 4u, 0x00020000);
+  const uint32_t srow = threadIdx.x / 32, scol = 4 * (threadIdx.x % 32);
+  const uint32_t stages = (p.d_model + kRouterStage - 1) / kRouterStage;
+  uint32_t next = q % stages;
+  struct Buf {
+    v4f v[4];
+    uint32_t k;
+  };
+  auto load = [&](Buf &b) {
+    b.k = kRouterStage * next + scol;
+    next = next + 1 == stages ? 0u : next + 1;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t o = b.k < p.d_model ? ((srow + 16 * (j % 2)) * p.d_model + b.k) * 4u : 0x80000000u;
+      b.v[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(j < 2 ? xr : gr, o, 0, 0));
+    }
+  };
+  auto store = [&](const Buf &b, uint32_t slab) {
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      v4f v = b.v[j];
+      if constexpr (!ALIGNED) {
+#pragma unroll
+        for (uint32_t i = 1; i < 4; ++i) v[i] = b.k + i < p.d_model ? v[i] : 0.f;
+      }
+      *reinterpret_cast<v4f *>(&lds[slab][srow + 16 * j][scol]) = v;
+    }
+  };
+  v4f part[4], sum[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[i] = sum[i] = v4f{0.f, 0.f, 0.f, 0.f};
+  Buf buf[2];
+  load(buf[0]);
+  load(buf[1]);
+  store(buf[0], 0);
+  load(buf[0]);
+  __syncthreads();
+  // stage s is in slab s % 2, s + 1 and s + 2 in buf (loads past the last
+  // stage repeat the first ones and are not used)
+  for (uint32_t s = 0; s < stages; s += 2) {
+#pragma unroll
+    for (uint32_t u = 0; u < 2; ++u) {
+      if (s + u >= stages) break;  // uniform
+      v4f in[4], t[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        in[i] = *reinterpret_cast<const v4f *>(&lds[u][16 * i + row][16 * wave + 4 * kg]);
+        t[i] = v4f{0.f, 0.f, 0.f, 0.f};
+      }
+      store(buf[u ^ 1], u ^ 1);
+      load(buf[u ^ 1]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)  // tile i: token half i / 2, expert half i % 2
+          t[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(in[i / 2][k], in[2 + i % 2][k], t[i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[i] += t[i];
+      __syncthreads();
+    }
+    if ((s & 7u) == 6u) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sum[i] += part[i];
+        part[i] = v4f{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  v4f(*red)[4][64] = reinterpret_cast<v4f(*)[4][64]>(lds);  // [wave][tile][lane]
+  static_assert(sizeof(lds) >= kRouterMWaves * 4 * 64 * sizeof(v4f), "the reduction fits in the stages' LDS");
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[wave][i][lane] = sum[i] + part[i];
+  __syncthreads();
+  if (wave >= 4) return;
+  v4f v = red[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < kRouterMWaves; ++w) v += red[w][wave][lane];
+  const uint32_t e = e0 + 16 * (wave % 2) + row;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t t = t0 + 16 * (wave / 2) + 4 * kg + i;
+    if (t < p.n_tokens && e < p.n_experts) p.logit_buf[(size_t)t * p.n_experts + e] = v[i];
+  }
+}
+
+// NPER: experts per lane, at least n_experts / 64.
+template <int NPER>
 __global__ __launch_bounds__(kSelThreads) void router_kernel(RouterParams p) {
   extern __shared__ float smem[];
   float *scores = smem;                               // [n_experts]
   float *selection = scores + p.n_experts;            // [n_experts]
   __shared__ float red_f[kSelWaves];
   __shared__ uint32_t group_ok[kMaxRouterExperts / 32];
-  __shared__ int32_t chosen[kMaxRouterTopK];
-  // thread 0's working arrays, in LDS (as private arrays they would live in
+  // the group filter's working arrays (thread 0's), in LDS (as private arrays they would live in
   // scratch memory, whose set-up dominates a launch this small)
   __shared__ int32_t sel_g[kMaxRouterGroups];  // surviving groups, best first
   __shared__ float sel_s[kMaxRouterGroups];
-  __shared__ float w[kMaxRouterTopK];
   __shared__ int32_t flag_bad;
 
   const uint32_t t = blockIdx.x;
@@ -234,45 +357,44 @@ __global__ __launch_bounds__(kSelThreads) void router_kernel(RouterParams p) {
   __syncthreads();
 
   // ---- top-k: k rounds of a wave arg-max -------------------------------
-  // Each round's winner (the largest packed candidate) is known to every
-  // lane; each lane remembers which of its own experts (lane, lane + 64, ...)
-  // are taken.
-  static_assert(kSelThreads == 64 && kMaxRouterExperts <= 64 * 64, "one wave, a 64-bit taken mask per lane");
-  uint64_t taken = 0;  // bit i: expert lane + 64 i is chosen
-  uint32_t count = 0;
-  for (uint32_t r = 0; r < p.top_k; ++r) {
-    uint64_t mine = 0;
-    uint32_t i = 0;
-    for (uint32_t e = lane; e < p.n_experts; e += 64, ++i) {
+  // Each lane keeps its experts' (lane, lane + 64, ...) packed candidates in
+  // registers; the winner of a round (the largest) is known to every lane and
+  // its owner drops it.
+  uint64_t cand[NPER];
+#pragma unroll
+  for (uint32_t i = 0; i < NPER; ++i) {
+    const uint32_t e = lane + 64 * i;
+    cand[i] = 0;
+    if (e < p.n_experts) {
       const float v = selection[e];
-      if (!__builtin_isfinite(v) || !((group_ok[e >> 5] >> (e & 31u)) & 1u) || ((taken >> i) & 1u)) continue;
-      const uint64_t c = pack_candidate(total_key(v), e);
-      mine = c > mine ? c : mine;
+      if (__builtin_isfinite(v) && ((group_ok[e >> 5] >> (e & 31u)) & 1u)) cand[i] = pack_candidate(total_key(v), e);
     }
+  }
+  uint32_t count = 0;
+  int32_t chosen = 0;  // lane r: the expert of round r
+  for (uint32_t r = 0; r < p.top_k; ++r) {
+    uint64_t mine = cand[0];
+#pragma unroll
+    for (uint32_t i = 1; i < NPER; ++i) mine = cand[i] > mine ? cand[i] : mine;
     const uint64_t best = wave_max_candidate(mine);
     if (best == 0) break;  // the same in every lane: no eligible expert left
-    const uint32_t bi = 0xffffffffu - (uint32_t)best;
-    if (lane == (bi & 63u)) taken |= 1ull << (bi >> 6);
-    if (lane == 0) chosen[r] = (int32_t)bi;
+#pragma unroll
+    for (uint32_t i = 0; i < NPER; ++i)
+      if (cand[i] == best) cand[i] = 0;
+    if (lane == r) chosen = (int32_t)(0xffffffffu - (uint32_t)best);
     count = r + 1;
   }
-  __syncthreads();
 
-  // ---- weights ------------------------------------------------------------
-  if (tid == 0) {
-    float sum = 0.f;
-    for (uint32_t i = 0; i < count; ++i) {
-      w[i] = scores[chosen[i]];
-      sum = sum + w[i];
-    }
-    if (p.normalise && __builtin_isfinite(sum) && sum > 0.f)
-      for (uint32_t i = 0; i < count; ++i) w[i] = w[i] / sum;
-    if (p.scaling != 1.0f && __builtin_isfinite(p.scaling))
-      for (uint32_t i = 0; i < count; ++i) w[i] = w[i] * p.scaling;
-    for (uint32_t i = 0; i < p.top_k; ++i) {
-      p.ids[(size_t)t * p.top_k + i] = i < count ? chosen[i] : -1;
-      p.weights[(size_t)t * p.top_k + i] = i < count ? w[i] : 0.0f;
-    }
+  // ---- weights: lane i's slot; the sum in slot order ------------------------
+  static_assert(kMaxRouterTopK <= 64, "one lane per slot");
+  float w = lane < count ? scores[chosen] : 0.f;
+  float sum = 0.f;
+  for (uint32_t i = 0; i < count; ++i) sum = sum + __shfl(w, (int)i, 64);
+  if (p.normalise && __builtin_isfinite(sum) && sum > 0.f) w = w / sum;
+  if (p.scaling != 1.0f && __builtin_isfinite(p.scaling)) w = w * p.scaling;
+  if (lane < p.top_k) {
+    p.ids[(size_t)t * p.top_k + lane] = lane < count ? chosen : -1;
+    p.weights[(size_t)t * p.top_k + lane] = lane < count ? w : 0.0f;
   }
 }
 
@@ -280,12 +402,24 @@ hipError_t launch_router(const RouterParams &p, hipStream_t st) {
   const uint32_t n_eg = (p.n_experts + kRouterWaves - 1) / kRouterWaves;
   const uint32_t n_tg = (p.n_tokens + kRouterTokGroup - 1) / kRouterTokGroup;
   const bool vec = p.d_model % 4 == 0 && (uintptr_t)p.gate % 16 == 0 && (uintptr_t)p.x % 16 == 0;
-  if (vec) hipLaunchKernelGGL(router_logits_kernel<true>, dim3(n_eg * n_tg), dim3(kRouterThreads), 0, st, p);
+  // One workgroup of the MFMA kernel takes ~1 us per 128 k-indices whatever
+  // the batch; the other kernel's time grows with tokens * experts.  Call us,
+  // that kernel / MFMA: 128 experts x 2048: 256 tokens 20 / 22, 512 tokens
+  // 32 / 23, 2048 tokens 101 / 25; 256 x 7168: 64 tokens 29 / 54, 2048 tokens
+  // 577 / 93; 160 x 3000, 300 tokens 55 / 46; 8 x 4096, 2048 tokens 26 / 35.
+  if ((uint64_t)p.n_tokens * p.n_experts >= 40000) {
+    const dim3 grid(8 * ((p.n_tokens + 8 * kRouterTile - 1) / (8 * kRouterTile)) * ((p.n_experts + kRouterTile - 1) / kRouterTile));
+    if (vec) hipLaunchKernelGGL(router_logits_mfma_kernel<true>, grid, dim3(64 * kRouterMWaves), 0, st, p);
+    else hipLaunchKernelGGL(router_logits_mfma_kernel<false>, grid, dim3(64 * kRouterMWaves), 0, st, p);
+  } else if (vec) hipLaunchKernelGGL(router_logits_kernel<true>, dim3(n_eg * n_tg), dim3(kRouterThreads), 0, st, p);
   else hipLaunchKernelGGL(router_logits_kernel<false>, dim3(n_eg * n_tg), dim3(kRouterThreads), 0, st, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const size_t lds = sizeof(float) * 2 * (size_t)p.n_experts;
-  hipLaunchKernelGGL(router_kernel, dim3(p.n_tokens), dim3(kSelThreads), lds, st, p);
+  const dim3 grid(p.n_tokens), block(kSelThreads);
+  if (p.n_experts <= 128) hipLaunchKernelGGL(router_kernel<2>, grid, block, lds, st, p);
+  else if (p.n_experts <= 256) hipLaunchKernelGGL(router_kernel<4>, grid, block, lds, st, p);
+  else hipLaunchKernelGGL(router_kernel<(int)kMaxRouterExperts / 64>, grid, block, lds, st, p);
   return hipGetLastError();
 }
 
