@@ -85,7 +85,7 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr uint32_t kBigTok = 64;             // pairs per token tile of gbig
-constexpr uint32_t kGMaxRun = 32;            // consecutive work items on one XCD (gbig)
+constexpr uint32_t kGMaxRun[2] = {8, 32};    // consecutive work items on one XCD (gbig: down, gate/up)
 constexpr uint32_t kNoLoad = 0x80000000u;    // an offset past every buffer: reads zeros
 
 // ---- gproj geometry -----------------------------------------------------
@@ -378,13 +378,13 @@ __global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
     const uint32_t nt = (c + kTile - 1) / kTile;
     cnt[e] = op;
     tcnt[e] = ot;
-    // 64-pair tiles of equal size, in whole groups of 16 pairs
-    const uint32_t size = kTile == kGTok || nt < 2 ? kTile : ((c + nt - 1) / nt + 15) / 16 * 16;
+    // full tiles, then the remainder: tiles of equal size are 4% slower at 512
+    // Mixtral tokens (a remainder of up to 32 pairs takes half the products)
     for (uint32_t j = 0; j < nt; ++j) {
       GroupTile t;
       t.blob = reinterpret_cast<const uint8_t *>(p.table[e]);
-      t.start = op + j * size;
-      t.count = min(size, c - j * size);
+      t.start = op + j * kTile;
+      t.count = min(kTile, c - j * kTile);
       p.tiles[ot + j] = t;
     }
     op += c;
@@ -755,15 +755,18 @@ __device__ __forceinline__ void wait_vm_barrier() {
 // the caller).  Items are ordered expert, token tile, row tile, and runs of
 // them go to one XCD: its workgroups then share one tile's inputs in their L2
 // (Mixtral prefill, 2048 tokens: 3.45 ms, 3.73 with the token tiles of a row
-// tile together).
+// tile together).  The down projection's items are fewer and longer (K parts
+// and d_model / 256 row tiles), so shorter runs end more evenly: with runs of
+// 8 it takes 325 us at 512 Mixtral tokens and 1.08 ms at 2048, with 32 363 us
+// and 1.11 ms; gate/up is 2-4% slower with runs of 8, 64 or 112.
 struct GItem {
   const uint8_t *blob;
   uint32_t start, count, rt;
 };
-__device__ __forceinline__ bool group_item(const GroupedParams &p, uint32_t row_tiles, GItem *it) {
+__device__ __forceinline__ bool group_item(const GroupedParams &p, uint32_t row_tiles, uint32_t max_run, GItem *it) {
   const uint32_t total = *p.n_tiles * row_tiles;
   const uint32_t x = blockIdx.x % 8, q = blockIdx.x / 8;
-  const uint32_t run = max(1u, min(total / 64, kGMaxRun));
+  const uint32_t run = max(1u, min(total / 64, max_run));
   const uint32_t item = ((q / run) * 8 + x) * run + q % run;
   if (item >= total) return false;
   const GroupTile gt = p.tiles[item / row_tiles];
@@ -1100,7 +1103,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   __shared__ __attribute__((aligned(16))) uint8_t lds[kX0 + kXSlots * kXSlot<MODE>];  // two workgroups per CU
   const uint32_t parts = FUSED ? 1u : p.n_parts;
   GItem it;
-  if (!group_item(p, ((FUSED ? 2 * p.d_ff : p.d_model) + kBigRows - 1) / kBigRows * parts, &it)) return;  // uniform
+  if (!group_item(p, ((FUSED ? 2 * p.d_ff : p.d_model) + kBigRows - 1) / kBigRows * parts, kGMaxRun[FUSED], &it)) return;  // uniform
   const uint32_t rt = it.rt / parts, part = it.rt % parts;
   if (it.count > 32) GBig<FMT, MODE, FUSED, 2>::run(p, it.blob, it.start, it.count, rt, part, lds);
   else GBig<FMT, MODE, FUSED, 1>::run(p, it.blob, it.start, it.count, rt, part, lds);
@@ -1228,7 +1231,7 @@ template <int FMT, int MODE, bool FUSED>
 static hipError_t launch_gbig(const GroupedParams &p, uint32_t max_tiles, hipStream_t st) {
   const uint32_t row_tiles = ((FUSED ? 2 * p.d_ff : p.d_model) + kBigRows - 1) / kBigRows * (FUSED ? 1u : p.n_parts);
   // whole runs of items on each XCD: up to one run per XCD past the items
-  const dim3 grid((max_tiles * row_tiles + 7) / 8 * 8 + 8 * kGMaxRun);
+  const dim3 grid((max_tiles * row_tiles + 7) / 8 * 8 + 8 * kGMaxRun[FUSED]);
   hipLaunchKernelGGL((gbig_kernel<FMT, MODE, FUSED>), grid, dim3(256), 0, st, p);
   return hipGetLastError();
 }
