@@ -97,7 +97,7 @@ struct DeviceState {
   int cus = 256;
   uint32_t *status = nullptr;
   uint64_t clock_khz = 100000;
-  std::atomic<int> occupancy[2][2][2][3][3] = {};  // resident decode workgroups per CU, by (Q8 act, pair, fmt, GG, GD)
+  std::atomic<int> occupancy[3][2][2][3][3] = {};  // resident decode workgroups per CU, by (mode, pair, fmt, GG, GD)
   // Device-wide order of persistent decode launches (guarded by
   // g_launch_mu).  The decode grid fills the device and hands items out by
   // static stride, so it needs all of its workgroups resident; two such
@@ -380,7 +380,7 @@ struct DecodePlan {
   int fmt;
   SliceGeom gg, gd;
   bool pair;  // two-wave workgroups: a tile's two gate/up slices add up in LDS
-  bool q8act;  // Q4_0 with Candle's Q8_0 activations (MER_MOE_QMM)
+  DecodeMode mode;
   size_t n_xd, n_gp, n_hd, n_pa;  // floats: x digit lines, gate/up slice partials, h digit lines, down partials
   size_t layer_flags, gd_flags;   // 64-bit release flags
   bool gd_fan;
@@ -392,7 +392,7 @@ void plan_decode(DecodePlan &pl, int dtype, size_t dm, size_t dff, uint32_t n_la
   DeviceState &dev = g_dev[g_device.load()];
   const int fmt = fmt_of(dtype);
   pl.fmt = fmt;
-  pl.q8act = fmt == FMT_Q4_0 && (flags & kFlagQ8Act) != 0;
+  pl.mode = flags & kFlagF16 ? kDecodeF16 : fmt == FMT_Q4_0 && (flags & kFlagQ8Act) ? kDecodeQ8Act : kDecodeF32;
   DecodeParams &p = pl.p;
   p = DecodeParams{};
   p.swiglu_limit = g_swiglu_limit.load();
@@ -445,7 +445,7 @@ void plan_decode(DecodePlan &pl, int dtype, size_t dm, size_t dff, uint32_t n_la
     return v && v[0] == '1';
   }();
   pl.pair = !no_pair && pl.gg.slices == 2 && pl.gg.G <= 32;
-  p.off_g = p.off_p + n_tok * p.p_items;
+  p.off_g = p.off_p + (flags & kFlagF16 ? 1u : n_tok) * p.p_items;
   if (pl.pair && (p.off_g & 1u)) ++p.off_g;  // one padding P item
   p.off_d = p.off_g + p.n_inst * p.g_slices * p.g_tiles;
   p.items_per_layer = p.off_d + p.n_inst * p.d_slices * p.d_tiles;
@@ -466,7 +466,7 @@ void plan_decode(DecodePlan &pl, int dtype, size_t dm, size_t dff, uint32_t n_la
 
   auto up64 = [](size_t v) { return (v + 63) / 64 * 64; };
   const size_t L = n_layers;
-  pl.n_xd = L * n_tok * p.xblocks * kLineDwords;
+  pl.n_xd = L * (flags & kFlagF16 ? 1u : n_tok) * p.xblocks * kLineDwords;
   pl.n_gp = p.g_slices > 1 && !pl.pair ? up64(L * p.n_inst * p.g_slices * 2 * dff) : 0;
   pl.n_hd = L * p.n_inst * p.hblocks * kLineDwords;
   pl.n_pa = up64(L * p.n_inst * p.d_slices * dm);
@@ -513,9 +513,9 @@ void bind_decode(DecodePlan &pl, float *f, uint32_t *counters, uint32_t *ctl, ui
 int launch_planned(DecodePlan &pl, hipStream_t st, const std::function<hipError_t()> &prep = nullptr) {
   DeviceState &dev = g_dev[g_device.load()];
   DecodeParams &p = pl.p;
-  const void *fn = decode_kernel_fn(pl.fmt, pl.gg.G, pl.gd.G, pl.pair, pl.q8act);
+  const void *fn = decode_kernel_fn(pl.fmt, pl.gg.G, pl.gd.G, pl.pair, pl.mode);
   const uint32_t wpg = pl.pair ? 2u : 1u;
-  std::atomic<int> &occ_slot = dev.occupancy[pl.q8act][pl.pair][pl.fmt][g_index(pl.gg.G)][g_index(pl.gd.G)];
+  std::atomic<int> &occ_slot = dev.occupancy[pl.mode][pl.pair][pl.fmt][g_index(pl.gg.G)][g_index(pl.gd.G)];
   int occ = occ_slot.load();
   if (occ == 0) {
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, 64 * wpg, 0);
@@ -1302,13 +1302,24 @@ int mer_hip_expert_batch_f16(int dtype, size_t d_model, size_t d_ff, size_t n_ex
   if (n_experts > (1u << 16) || table_len > UINT32_MAX)
     return fail(MER_ERR_SHAPE_EXCEEDS_WORKSPACE, "too many experts in one batch");
   if (!d_expert_table || !d_expert_ids || !d_x || !d_out) return fail(MER_ERR_INVALID_LAYOUT, "null device pointer");
-  // Each expert is a one-slot token of weight 1 on its own copy of x, so
-  // the routed forward's output row i is y of expert i, uncombined.
+  // Each expert is a one-slot token of weight 1, so the routed forward's
+  // output row i is y of expert i, uncombined.  The decode kernel reads and
+  // writes the f16 itself; sizes it does not take are staged through f32,
+  // each expert on its own copy of x.
   const hipStream_t st = (hipStream_t)stream;
   std::shared_ptr<Workspace> w = workspace_for(st);
   if (!w) return require_init();
   std::lock_guard<std::mutex> wl(w->mu);
   if (w->released) return released_error();
+  if (decode_eligible(d_model, d_ff, nullptr)) {
+    LayerArgs la{};
+    la.table = d_expert_table;
+    la.table_len = (uint32_t)table_len;
+    la.ids = d_expert_ids;
+    la.x = reinterpret_cast<const float *>(d_x);
+    la.out = reinterpret_cast<float *>(d_out);
+    return run_decode(*w, dtype, d_model, d_ff, 1u, (uint32_t)n_experts, 1u, &la, nullptr, kFlagF16);
+  }
   const size_t need = 2 * n_experts * d_model;
   rc = ensure_buf(*w, &w->stage, &w->stage_floats, need, 0, false, "f16 staging allocation");
   if (rc) return rc;

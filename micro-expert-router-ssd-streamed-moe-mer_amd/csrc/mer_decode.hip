@@ -285,9 +285,10 @@ __device__ __forceinline__ float span_sum(float v) {
 // Quantise `nblocks` (<= 64 / groups) blocks of x into digit planes in line
 // format (dword 24 = scale, dwords 25..26 = launch epoch); one wave, lane =
 // group.  DEV: x is read with device-scope loads (it may have been written
-// by another wave of this launch); otherwise x is in LDS.
-template <int FMT, bool DEV, bool Q8ACT = false>
-__device__ __forceinline__ void pack_blocks(const float *x, uint32_t nblocks, uint32_t *dig, uint64_t epoch) {
+// by another wave of this launch); otherwise x is in LDS, or the caller's
+// f16 vector.
+template <int FMT, bool DEV, bool Q8ACT = false, typename T>
+__device__ __forceinline__ void pack_blocks(const T *x, uint32_t nblocks, uint32_t *dig, uint64_t epoch) {
   using D = DigitTraits<FMT>;
   const uint32_t g = lane_id();
   const bool valid = g < nblocks * D::kGroups;
@@ -296,11 +297,12 @@ __device__ __forceinline__ void pack_blocks(const float *x, uint32_t nblocks, ui
   float amax = 0.f;
   int finite = 1;
   if (valid) {
-    const float *xb = x + (size_t)b * 32;
+    const T *xb = x + (size_t)b * 32;
 #pragma unroll
     for (int i = 0; i < D::kGroupElems; ++i) {
-      const float *src = xb + group_elem<FMT>((int)m, i);
-      v[i] = DEV ? ld_dev(src) : *src;
+      const T *src = xb + group_elem<FMT>((int)m, i);
+      if constexpr (DEV) v[i] = ld_dev(src);
+      else v[i] = (float)*src;
     }
 #pragma unroll
     for (int i = 0; i < D::kGroupElems; ++i) {
@@ -516,8 +518,16 @@ __device__ __forceinline__ void fetch_digits(const uint32_t *dig, size_t block0,
 // experts): the slices of a tile are consecutive items, so they meet in one
 // workgroup and their partial sums are added in LDS instead of going
 // through memory and an arrival count (one round trip instead of three).
-template <int FMT, int GG, int GD, bool PAIR, bool Q8ACT>
+//
+// MODE kDecodeF16: the one layer of a call on f16 views.  Every token reads
+// one f16 input vector, packed once by the first token's P items, and the
+// combine writes f16.  A combine runs after all P items, so the output may
+// lie on the input.  A kernel of its own: the branches as a run-time flag
+// cost the other modes 0.1 us per launch, the conversions as launches before
+// and after it 6 us of 30 (8 Qwen3 experts, 24 us here).
+template <int FMT, int GG, int GD, bool PAIR, int MODE>
 __global__ __launch_bounds__(PAIR ? 128 : 64) __attribute__((amdgpu_waves_per_eu(FMT == FMT_Q4_0 ? 3 : 2))) void decode_kernel(DecodeParams p) {
+  constexpr bool Q8ACT = MODE == kDecodeQ8Act, kF16 = MODE == kDecodeF16;
   constexpr uint32_t kW = PAIR ? 2 : 1;  // waves per workgroup
   const uint32_t wv = PAIR ? (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / 64) : 0u;
   __shared__ float s_h_all[kW][kTileRows];
@@ -566,6 +576,7 @@ __global__ __launch_bounds__(PAIR ? 128 : 64) __attribute__((amdgpu_waves_per_eu
     auto wait_prev_layer = [&](uint32_t t) {
       if (l > 0) wait_flag(p, release_flag(p, l - 1, t, (uint32_t)(gi % kReleaseFan)), epoch, kNapFlag);
     };
+    auto input_of = [&](uint32_t t) { return kF16 ? 0u : t; };  // the input vector of token t
     const bool route_after_prev = (p.flags & kFlagRouteAfterPrev) != 0;
     // Layer l's input digits of token t are complete.  Layer 0's are packed
     // by its P items; with combine packing, layer l > 0's input block b is
@@ -573,7 +584,7 @@ __global__ __launch_bounds__(PAIR ? 128 : 64) __attribute__((amdgpu_waves_per_eu
     // once every tile of layer l-1 is combined.
     auto wait_input = [&](uint32_t t) {
       if (l > 0 && p.combine_packs) wait_prev_layer(t);
-      else wait_for(p, cnt + p.c_p + (size_t)t * kPollStride, p.p_items, kNapCounter);
+      else wait_for(p, cnt + p.c_p + (size_t)input_of(t) * kPollStride, p.p_items, kNapCounter);
     };
     // Under ROUTE_AFTER_PREV, G and D items touch their experts only once the
     // layer's input is packed (which implies layer l-1 is complete), so the
@@ -601,13 +612,16 @@ __global__ __launch_bounds__(PAIR ? 128 : 64) __attribute__((amdgpu_waves_per_eu
       const uint32_t idx = j - p.off_p;
       const uint32_t t = idx / p.p_items;
       const uint32_t part = idx % p.p_items;
-      if (t < p.n_tok && (l == 0 || !p.combine_packs)) {  // else packed by layer l-1's combines (or padding)
+      if (t < (kF16 ? 1u : p.n_tok) && (l == 0 || !p.combine_packs)) {  // else packed by layer l-1's combines (or padding)
         wait_prev_layer(t);  // layers run in order: layer l reads after layer l-1 wrote
         tm.ready = trace_now(p);
         const uint32_t b0 = part * kPackBlocks;
         const uint32_t nb = min(kPackBlocks, p.xblocks - b0);
         const size_t tb = (size_t)t * p.xblocks + b0;
-        pack_blocks<FMT, true, Q8ACT>(xsrc + (size_t)t * p.d_model + (size_t)b0 * 32, nb, xq_dig + tb * kLineDwords, epoch);
+        if constexpr (kF16)
+          pack_blocks<FMT, false, Q8ACT>(reinterpret_cast<const _Float16 *>(xsrc) + (size_t)b0 * 32, nb, xq_dig + tb * kLineDwords, epoch);
+        else
+          pack_blocks<FMT, true, Q8ACT>(xsrc + (size_t)t * p.d_model + (size_t)b0 * 32, nb, xq_dig + tb * kLineDwords, epoch);
         signal(cnt + p.c_p + (size_t)t * kPollStride);
       }
     } else if (j < p.off_d) {
@@ -636,7 +650,7 @@ __global__ __launch_bounds__(PAIR ? 128 : 64) __attribute__((amdgpu_waves_per_eu
       uint32_t xd[2 * kBlockDigitDwords];
       float xsc[2];
       prio_hi();
-      fetch_digits(xq_dig, (size_t)t * p.xblocks + 2 * (size_t)c, valid, epoch, xd, xsc);
+      fetch_digits(xq_dig, (size_t)input_of(t) * p.xblocks + 2 * (size_t)c, valid, epoch, xd, xsc);
       prio_lo();
       tm.fetched = trace_now(p);
       float *gpart = p.gpart + (((size_t)l * p.n_inst + inst) * p.g_slices + gs) * 2 * p.d_ff;
@@ -776,7 +790,8 @@ __global__ __launch_bounds__(PAIR ? 128 : 64) __attribute__((amdgpu_waves_per_eu
             for (uint32_t k = 0; k < n_parts; ++k) acc += ld_dev(pp + (size_t)k * p.d_model);
           }
           const float val = (p.flags & (kFlagResidual | kFlagAccumulate)) ? base + acc : acc;
-          st_dev(o, val);
+          if constexpr (kF16) reinterpret_cast<_Float16 *>(la.out)[(size_t)t * p.d_model + r] = (_Float16)val;
+          else st_dev(o, val);
           if (pack_next) s_h[lane] = (p.flags & kFlagChain) ? val : next_x;
         }
         if (pack_next) {
@@ -848,32 +863,34 @@ hipError_t launch_decode_scratch_prep(uint32_t *ctl, uint32_t n_ctl, uint32_t *z
   return hipGetLastError();
 }
 
-template <int FMT, int GG, int GD, bool PAIR, bool Q8ACT>
+template <int FMT, int GG, int GD, bool PAIR, int MODE>
 static const void *decode_fn() {
-  return reinterpret_cast<const void *>(&decode_kernel<FMT, GG, GD, PAIR, Q8ACT>);
+  return reinterpret_cast<const void *>(&decode_kernel<FMT, GG, GD, PAIR, MODE>);
 }
 
-template <int FMT, int GG, bool PAIR, bool Q8ACT>
+template <int FMT, int GG, bool PAIR, int MODE>
 static const void *decode_fn_gd(int gd) {
-  if (gd == 16) return decode_fn<FMT, GG, 16, PAIR, Q8ACT>();
-  if (gd == 32) return decode_fn<FMT, GG, 32, PAIR, Q8ACT>();
-  return decode_fn<FMT, GG, 64, PAIR, Q8ACT>();
+  if (gd == 16) return decode_fn<FMT, GG, 16, PAIR, MODE>();
+  if (gd == 32) return decode_fn<FMT, GG, 32, PAIR, MODE>();
+  return decode_fn<FMT, GG, 64, PAIR, MODE>();
 }
 
 // Paired workgroups serve gate/up rows cut into two slices of at most 32
 // chunks (GG 16 or 32); single-wave workgroups serve everything else.
-template <int FMT, bool Q8ACT>
+template <int FMT, int MODE>
 static const void *decode_fn_fmt(int gg, int gd, bool pair) {
-  if (pair) return gg == 16 ? decode_fn_gd<FMT, 16, true, Q8ACT>(gd) : decode_fn_gd<FMT, 32, true, Q8ACT>(gd);
-  if (gg == 16) return decode_fn_gd<FMT, 16, false, Q8ACT>(gd);
-  if (gg == 32) return decode_fn_gd<FMT, 32, false, Q8ACT>(gd);
-  return decode_fn_gd<FMT, 64, false, Q8ACT>(gd);
+  if (pair) return gg == 16 ? decode_fn_gd<FMT, 16, true, MODE>(gd) : decode_fn_gd<FMT, 32, true, MODE>(gd);
+  if (gg == 16) return decode_fn_gd<FMT, 16, false, MODE>(gd);
+  if (gg == 32) return decode_fn_gd<FMT, 32, false, MODE>(gd);
+  return decode_fn_gd<FMT, 64, false, MODE>(gd);
 }
 
-// q8act: Candle's Q8_0 activations (QMatMul), Q4_0 weights only.
-const void *decode_kernel_fn(int fmt, int gg, int gd, bool pair, bool q8act) {
-  if (fmt != FMT_Q4_0) return decode_fn_fmt<FMT_Q8_0, false>(gg, gd, pair);
-  return q8act ? decode_fn_fmt<FMT_Q4_0, true>(gg, gd, pair) : decode_fn_fmt<FMT_Q4_0, false>(gg, gd, pair);
+const void *decode_kernel_fn(int fmt, int gg, int gd, bool pair, DecodeMode mode) {
+  if (fmt != FMT_Q4_0)
+    return mode == kDecodeF16 ? decode_fn_fmt<FMT_Q8_0, kDecodeF16>(gg, gd, pair) : decode_fn_fmt<FMT_Q8_0, kDecodeF32>(gg, gd, pair);
+  if (mode == kDecodeF16) return decode_fn_fmt<FMT_Q4_0, kDecodeF16>(gg, gd, pair);
+  return mode == kDecodeQ8Act ? decode_fn_fmt<FMT_Q4_0, kDecodeQ8Act>(gg, gd, pair)
+                              : decode_fn_fmt<FMT_Q4_0, kDecodeF32>(gg, gd, pair);
 }
 
 hipError_t launch_decode(const void *fn, uint32_t grid, uint32_t waves_per_group, const DecodeParams &p,
