@@ -98,3 +98,37 @@ def test_tiles_extreme_inputs(mer, oracle, gpu):
         assert np.abs(got[t] - want).max() <= 1e-5 * np.abs(want).max(), t
     mer.take_device_status()
     del devs
+
+
+@pytest.mark.parametrize("table_len,n_tok,k", [(1, 5, 1), (1024, 171, 6), (1025, 170, 6), (4096, 200, 7)])
+def test_grouping_sparse_table(mer, oracle, gpu, table_len, n_tok, k):
+    """Grouping with one and several experts and pairs per thread: absent
+    entries, negative ids and ids past the table are misses, zero-weight
+    slots are skipped whatever their id."""
+    dm = dff = 64
+    say(f"grouping table={table_len} tokens={n_tok} k={k}")
+    blobs = [make_expert(oracle, Q8, dm, dff, 30 + e) for e in range(3)]
+    devs, base = _table(blobs, gpu)
+    rng = np.random.default_rng(table_len)
+    kind = np.arange(table_len) % 4  # 3: absent
+    table = torch.where(torch.from_numpy(kind == 3).to(gpu), torch.zeros(1, dtype=torch.int64, device=gpu),
+                        base[torch.from_numpy(kind % 3).to(gpu)])
+    ids = rng.integers(-2, table_len + 2, (n_tok, k)).astype(np.int32)
+    w = rng.random((n_tok, k)).astype(np.float32) + np.float32(0.1)
+    w[rng.random((n_tok, k)) < 0.2] = 0.0
+    x = rng.standard_normal((n_tok, dm)).astype(np.float32)
+    want = np.zeros((n_tok, dm), np.float32)
+    for t in range(n_tok):
+        valid = [j for j in range(k) if 0 <= ids[t, j] < table_len and kind[ids[t, j]] != 3 and w[t, j] != 0]
+        if valid:
+            ys = [oracle.q8_0_direct_forward(blobs[kind[ids[t, j]] % 3], x[t], dm, dff)[1] for j in valid]
+            want[t] = oracle.combine_outputs(np.stack(ys), w[t, valid])
+    got = mer.moe_grouped(mer.WeightDtype.Q8_0, dm, dff, table, to_dev(ids, gpu), to_dev(w, gpu), to_dev(x, gpu))
+    got = got.cpu().numpy()
+    missed = (w != 0) & ((ids < 0) | (ids >= table_len) | (kind[np.clip(ids, 0, table_len - 1)] == 3))
+    if missed.any():
+        with pytest.raises(mer.GpuExpertDispatchError):
+            mer.take_device_status()
+    mer.take_device_status()
+    assert_ffn_close(got, want, "sparse table")
+    del devs
