@@ -48,7 +48,7 @@
  *     with MER_ERR_PHYSICAL_CAPACITY).  Replays are correct: the decode
  *     kernel's epoch lives in device memory and each launch hands the
  *     next one a fresh value.  A captured graph holds the workspace's
- *     buffer addresses: a later call of a larger shape on that stream
+ *     buffer addresses: a later call larger in any size on that stream
  *     (which grows the workspace) or mer_hip_stream_release invalidates
  *     graphs captured on it.  Captured decode launches are not ordered
  *     against decode calls on other streams; the caller orders replays.

@@ -14,7 +14,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "libmer_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["mer_kernels.hip", "mer_decode.hip", "mer_router.hip", "mer_grouped.hip", "mer_slots.hip", "mer_format.cpp", "mer_abi.hip"]
-HEADERS = ["mer_device.hpp", "mer_internal.hpp"]
+HEADERS = ["mer_device.hpp", "mer_internal.hpp", "mer_grouped_plan.hpp"]
 
 HIPCC_FLAGS = [
     "-std=c++17",

@@ -79,6 +79,7 @@ struct Workspace {
   hipStream_t stream = nullptr;
   float *scratch = nullptr;      // h vectors, digit lines, partial sums
   size_t scratch_floats = 0;
+  size_t scratch_refused = SIZE_MAX;  // smallest size that could only be wished for (ensure_scratch_upto)
   float *stage = nullptr;        // f32 x and y of the f16-view entry point
   size_t stage_floats = 0;
   float *router_buf = nullptr;   // router logits when the caller asks for none
@@ -219,6 +220,7 @@ void free_workspace(Workspace &w) {
   w.scratch = w.stage = w.router_buf = nullptr;
   w.counters = nullptr;
   w.release = nullptr;
+  w.scratch_refused = SIZE_MAX;
   w.scratch_floats = w.stage_floats = w.router_floats = w.counter_words = w.release_words = 0;
 }
 
@@ -262,6 +264,33 @@ int ensure_scratch(Workspace &w, size_t floats, float **out) {
   int rc = ensure_buf(w, &w.scratch, &w.scratch_floats, floats, size_t(1) << 20, false, "scratch allocation");
   *out = w.scratch;
   return rc;
+}
+
+// At least `need` floats, and `want` where the device has them outside
+// capture.  The buffer in use is given up only for a larger one at hand, so a
+// device too full for `want` still serves what `need` covers; a size once
+// refused is not asked for again.
+int ensure_scratch_upto(Workspace &w, size_t need, size_t want, float **out) {
+  if (w.scratch_floats < want && want < w.scratch_refused && !capturing(w.stream)) {
+    const size_t floats = want < (size_t(1) << 20) ? size_t(1) << 20 : want;
+    float *buf = nullptr;
+    if (hipMalloc(reinterpret_cast<void **>(&buf), floats * sizeof(float)) != hipSuccess) {
+      (void)hipGetLastError();  // the next launch's check must not see it
+      w.scratch_refused = want;
+    } else {
+      if (w.scratch) {
+        const hipError_t e = hipStreamSynchronize(w.stream);
+        if (e != hipSuccess) {
+          (void)hipFree(buf);
+          return hip_fail(e, MER_ERR_DEVICE_LOST, "synchronise before workspace growth");
+        }
+        (void)hipFree(w.scratch);
+      }
+      w.scratch = buf;
+      w.scratch_floats = floats;
+    }
+  }
+  return ensure_scratch(w, need, out);
 }
 
 // Decode counters: `words` per launch plus the control lines, all zero
@@ -819,69 +848,23 @@ int run_grouped(Workspace &w, int dtype, size_t dm, size_t dff, uint32_t n_token
   p.hblocks = (uint32_t)(dff / 32);
   p.proj_bytes = div_ceil(dm * dff, 32) * block_bytes(dtype);
   p.status = dev.status;
-  const uint32_t max_experts = p.n_pairs < table_len ? p.n_pairs : table_len;
-  // Tiles of 64 pairs on f16 MFMA (gbig) from 16 pairs per expert on average,
-  // or 8 where the experts alone give the 512 resident workgroups four
-  // rounds; else the int8 kernel's tiles of 16.  Call us, int8 / f16, at 8
-  // pairs: Qwen3 Q8_0 138 / 158, Mixtral Q4_0 282 / 287, DeepSeek-V3 Q4_0
-  // (4096 workgroups) 1424 / 1119; at 16 pairs: 208 / 207, 434 / 302, 2290 /
-  // 1600; Mixtral under MER_MOE_QMM at 8 and 16: 279 / 331, 433 / 342.
-  const size_t expert_wgs = (size_t)max_experts * div_ceil(2 * dff, 256);
-  const bool big = p.n_pairs >= 16 * max_experts || (p.n_pairs >= 8 * max_experts && expert_wgs >= 2048);
-  p.mode = !big ? kGroupDigits : p.q8act ? kGroupQ8Act : kGroupF16Pair;
-  const uint32_t tile_pairs = big ? 64u : 16u;
-  // Down rows in up to 4 K parts (whole 4-block stages, about 64 blocks or
-  // more) until 2048 workgroups share the launch: 512 run at once, and a short
-  // last round of whole rows idles the chip.  Mixtral Q4_0 down, us with one
-  // part / with parts: 64 tokens 195 / 94, 128 tokens 281 / 119, 2048 tokens
-  // 1200 / 1105 (combine 20 / 33).
-  p.n_parts = 1;
-  p.part_blocks = p.hblocks;
-  if (big) {
-    const uint32_t wgs = (p.n_pairs / tile_pairs + (max_experts + 1) / 2) * (uint32_t)div_ceil(dm, 256);
-    while (p.n_parts < 4 && wgs * p.n_parts < 2048 && p.hblocks >= 128 * p.n_parts) p.n_parts *= 2;
-    p.part_blocks = (uint32_t)div_ceil(p.hblocks, 4 * p.n_parts) * 4;
-    p.n_parts = (uint32_t)div_ceil(p.hblocks, p.part_blocks);
-  }
-  // At most n_pairs / tile_pairs full tiles plus one partial tile per
-  // distinct expert.
-  const uint32_t max_tiles = p.n_pairs / tile_pairs + max_experts;
-
-  auto up64 = [](size_t v) { return (v + 63) / 64 * 64; };  // floats; 256-byte aligned regions
-  const size_t n_hdr = 64;
-  const size_t n_plist = up64(p.n_pairs);
-  const size_t n_ok = up64(p.n_pairs);
-  const size_t n_tiles = up64((size_t)max_tiles * sizeof(GroupTile) / 4);
-  const size_t rec = p.mode == kGroupQ8Act ? 16 : 32;  // record dwords per block
-  const size_t n_xg = up64((size_t)n_tokens * p.xblocks * rec);
-  const size_t n_hg = up64((size_t)p.n_pairs * p.hblocks * rec);
-  const size_t n_xs = big ? up64((size_t)n_tokens * p.xblocks) : 0;
-  const size_t n_hs = big ? up64((size_t)p.n_pairs * p.hblocks) : 0;
-  const size_t n_h32 = big ? up64((size_t)p.n_pairs * dff) : 0;
-  const size_t n_pa = up64((size_t)p.n_parts * p.n_pairs * dm);
-  const size_t total = n_h32 + n_hdr + n_plist + n_ok + n_tiles + n_xg + n_hg + n_xs + n_hs + n_pa;
-  float *cur = nullptr;
-  int rc = ensure_scratch(w, total, &cur);
+  GroupedPlan pl = plan_grouped(p.q8act != 0, dm, dff, n_tokens, top_k, table_len);
+  float *f = nullptr;
+  int rc = ensure_scratch_upto(w, pl.need, pl.want, &f);
   if (rc) return rc;
-  p.n_tiles = reinterpret_cast<uint32_t *>(cur);
-  cur += n_hdr;
-  p.plist = reinterpret_cast<uint32_t *>(cur);
-  cur += n_plist;
-  p.pair_ok = reinterpret_cast<uint32_t *>(cur);
-  cur += n_ok;
-  p.tiles = reinterpret_cast<GroupTile *>(cur);
-  cur += n_tiles;
-  p.xg = reinterpret_cast<uint32_t *>(cur);
-  cur += n_xg;
-  p.hg = reinterpret_cast<uint32_t *>(cur);
-  cur += n_hg;
-  p.xs = cur;
-  cur += n_xs;
-  p.hs = cur;
-  cur += n_hs;
-  p.h32 = cur;
-  cur += n_h32;
-  p.partial = cur;
+  fit_parts(pl, p.n_pairs, dm, dff, w.scratch_floats);
+  p.mode = pl.mode;
+  p.n_parts = pl.n_parts;
+  p.part_blocks = pl.part_blocks;
+  p.n_tiles = reinterpret_cast<uint32_t *>(f);
+  p.plist = reinterpret_cast<uint32_t *>(f + pl.plist);
+  p.pair_ok = reinterpret_cast<uint32_t *>(f + pl.pair_ok);
+  p.tiles = reinterpret_cast<GroupTile *>(f + pl.tiles);
+  p.xg = reinterpret_cast<uint32_t *>(f + pl.xg);
+  p.hg = reinterpret_cast<uint32_t *>(f + pl.hg);
+  p.xs = f + pl.xs;
+  p.hs = f + pl.hs;
+  p.partial = f + pl.partial;
 
   const int fmt = fmt_of(dtype);
   size_t tl = SIZE_MAX;
@@ -891,11 +874,11 @@ int run_grouped(Workspace &w, int dtype, size_t dm, size_t dff, uint32_t n_token
   if ((e = launch_grouped_prep(fmt, p, st)) != hipSuccess) return hip_fail(e, MER_ERR_SUBMISSION, "grouping launch");
   if ((trc = timing_end(tl, st))) return trc;
   if ((trc = timing_begin(STAGE_GATE_UP, st, &tl))) return trc;
-  if ((e = launch_grouped_proj(fmt, true, p, max_tiles, st)) != hipSuccess)
+  if ((e = launch_grouped_proj(fmt, true, p, pl.max_tiles, st)) != hipSuccess)
     return hip_fail(e, MER_ERR_SUBMISSION, "grouped gate/up launch");
   if ((trc = timing_end(tl, st))) return trc;
   if ((trc = timing_begin(STAGE_DOWN, st, &tl))) return trc;
-  if ((e = launch_grouped_proj(fmt, false, p, max_tiles, st)) != hipSuccess)
+  if ((e = launch_grouped_proj(fmt, false, p, pl.max_tiles, st)) != hipSuccess)
     return hip_fail(e, MER_ERR_SUBMISSION, "grouped down launch");
   if ((trc = timing_end(tl, st))) return trc;
   if ((trc = timing_begin(STAGE_COMBINE, st, &tl))) return trc;

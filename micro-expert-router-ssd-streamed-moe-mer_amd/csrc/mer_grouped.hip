@@ -112,6 +112,7 @@ struct GGeom {
 };
 constexpr float kGIntMax = 8355711.0f;   // |v| bound (0x7f7f7f): v + 0x808080 stays in 24 bits
 constexpr uint32_t kGRec = 8;            // dwords per (vector, block, k-group) record: 3 digit planes, scale, pad
+static_assert(4 * kGRec == kGroupRecDwords, "four k-groups a block");
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 
@@ -194,10 +195,11 @@ __device__ __forceinline__ constexpr uint32_t kgroup_elem(uint32_t m, int i) {
   }
 }
 
-// One Q8_0-activation record: 8 elements (in kgroup_elem order) of a block
-// whose 4 groups sit in 4 adjacent lanes (lane & 3 = group m), and the
-// block's scale.  Only lanes with `store` write.
-__device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint4 *rec, float *scale, uint32_t m, bool store) {
+// One k-group of a Q8_0-activation record (the four groups' 16 bytes, then
+// the block's f32 scale): 8 elements (in kgroup_elem order) of a block whose
+// 4 groups sit in 4 adjacent lanes (lane & 3 = group m).  Only lanes with
+// `store` write.
+__device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint4 *rec, uint32_t m, bool store) {
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[i]));
@@ -208,8 +210,8 @@ __device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint4 *rec, 
   v8h q;
 #pragma unroll
   for (int i = 0; i < 8; ++i) q[i] = (_Float16)quantize_elem_q8(v[i], bs.inv);
-  *rec = __builtin_bit_cast(uint4, q);
-  if (m == 0) *scale = bs.s;
+  rec[m] = __builtin_bit_cast(uint4, q);
+  if (m == 0) *reinterpret_cast<float *>(rec + 4) = bs.s;
 }
 
 // Eight elements of block b, k-group m of the f32 vector x, in kgroup_elem order.
@@ -231,7 +233,8 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 // kF16Pair records (per block the four k-groups' high parts, then their low
 // parts) and scale of one f32 vector of `blocks` blocks, by the whole
 // workgroup; a non-finite vector gets a NaN scale.  Two passes over x: the
-// second reads caches.
+// second reads caches.  The records may lie on x: a block is read and written
+// by four lanes of one wave, and the stores need all of the block's loads.
 template <int FMT>
 __device__ __forceinline__ void quant_vector(const float *x, uint32_t blocks, uint4 *rec, float *scale) {
   __shared__ float red[16];
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
       float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if constexpr (MODE == kQ8Act) {
         if (valid) load_group<FMT>(p.x, tb, m, v);
-        quant_group_q8(v, reinterpret_cast<uint4 *>(p.xg) + (size_t)tb * 4 + m, p.xs + tb, m, valid);
+        quant_group_q8(v, reinterpret_cast<uint4 *>(p.xg) + (size_t)tb * 8, m, valid);
       } else {
         if (valid) load_group<FMT_Q8_0>(p.x, tb, m, v);  // eight consecutive elements
         quant_group(v, p.xg + ((size_t)tb * 4 + m) * kGRec, valid, p.q8act != 0);
@@ -806,6 +809,7 @@ constexpr uint32_t kBigStride = 16 * kBigGran;
 constexpr uint32_t kBigSlab = kBigRows * kBigStride;
 constexpr uint32_t kXSlots = 5;
 constexpr uint32_t kX0 = 2 * kBigSlab;                    // LDS offset of the input slots
+constexpr uint32_t kRecBytes = 4 * kGroupRecDwords;       // a block's record in memory
 // LDS bytes of a block of 64 pairs' inputs: records, or records and scales
 template <int MODE> constexpr uint32_t kXSlot = MODE == kF16Pair ? 64 * 128 : 64 * 64 + 4 * 256;
 
@@ -867,26 +871,21 @@ struct GBig {
     // copies k-group l / 16 of vector l % 16 (64 contiguous bytes per
     // vector).  Wave w makes copies w, w + 4 (of 2 NG kParts; where there are
     // fewer than four, waves repeat them).
-    const uint32_t vec_bytes = row_blocks * 64u * kParts;
+    const uint32_t vec_bytes = row_blocks * kRecBytes;
     const uint32_t n_vec = FUSED ? p.n_tok : p.n_pairs;
     const uint64_t xbase = reinterpret_cast<uint64_t>(FUSED ? p.xg : p.hg);
     const v4u xr = {(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)xbase),
                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(xbase >> 32)), n_vec * vec_bytes, 0x00020000u};
     uint32_t xoff[kXCopies], soff = kNoLoad;
-    v4u sr = xr;
-    if constexpr (MODE == kQ8Act) {
-      const uint64_t sbase = reinterpret_cast<uint64_t>(FUSED ? p.xs : p.hs);
-      sr = v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)sbase),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(sbase >> 32)), n_vec * row_blocks * 4u, 0x00020000u};
-    }
 #pragma unroll
     for (int j = 0; j < kXCopies; ++j) {
       const uint32_t i = (wave + 4u * j) % (2 * NG * kParts);
       const uint32_t n = 16 * (i / kParts) + lane % 16;
       const uint32_t pair = n < count ? p.plist[start + n] : 0u;
       // a column without a pair reads zeros
-      xoff[j] = n < count ? (FUSED ? pair / p.top_k : pair) * vec_bytes + b0 * 64u * kParts + 64u * (i % kParts) + 16u * (lane / 16) : kNoLoad;
-      if (MODE == kQ8Act && n < count) soff = ((FUSED ? pair / p.top_k : pair) * row_blocks + b0) * 4u;
+      const uint32_t rec = (FUSED ? pair / p.top_k : pair) * vec_bytes + b0 * kRecBytes;
+      xoff[j] = n < count ? rec + 64u * (i % kParts) + 16u * (lane / 16) : kNoLoad;
+      if (MODE == kQ8Act && n < count) soff = rec + 64u;
     }
     uint32_t x_issued = 0, x_slot = 0;
     auto issue_x = [&]() {
@@ -894,11 +893,11 @@ struct GBig {
 #pragma unroll
       for (int j = 0; j < kXCopies; ++j) {
         async_lds16(xr, xoff[j] | none, lds0 + kX0 + x_slot * kXSlot<MODE> + (wave + 4u * j) % (2 * NG * kParts) * 1024u);
-        xoff[j] += 64u * kParts;
+        xoff[j] += kRecBytes;
       }
       if constexpr (MODE == kQ8Act) {  // the scales of the copy's 16 vectors, four times over
-        async_lds4(sr, soff | none, lds0 + kX0 + x_slot * kXSlot<MODE> + 4096u + wave % (2 * NG) * 256u);
-        soff += 4u;
+        async_lds4(xr, soff | none, lds0 + kX0 + x_slot * kXSlot<MODE> + 4096u + wave % (2 * NG) * 256u);
+        soff += kRecBytes;
       }
       ++x_issued;
       x_slot = x_slot + 1 == kXSlots ? 0u : x_slot + 1;
@@ -1080,7 +1079,7 @@ struct GBig {
     float *pscale = reinterpret_cast<float *>(lds + 64 * 8);
     if (tid < 32 * NG && tid < count) {
       const uint32_t pr = p.plist[start + tid];
-      prow[tid] = reinterpret_cast<uint64_t>(FUSED ? p.h32 + (size_t)pr * p.d_ff : p.partial + ((size_t)part * p.n_pairs + pr) * p.d_model);
+      prow[tid] = reinterpret_cast<uint64_t>(FUSED ? reinterpret_cast<float *>(p.hg) + (size_t)pr * p.d_ff : p.partial + ((size_t)part * p.n_pairs + pr) * p.d_model);
       const float sc = MODE == kQ8Act ? 1.0f : FUSED ? p.xs[pr / p.top_k] : p.hs[pr];  // the vector's scale
       pscale[tid] = !FUSED && p.weights ? sc * p.weights[pr] : sc;
     }
@@ -1116,21 +1115,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   else GBig<FMT, MODE, FUSED, 1>::run(p, it.blob, it.start, it.count, rt, part, lds);
 }
 
-// The records of h for gbig's down projection, one workgroup per routed pair.
+// The records of h for gbig's down projection, in h's place, one workgroup per
+// routed pair.
 template <int FMT, int MODE>
 __global__ __launch_bounds__(256) void hquant_kernel(GroupedParams p) {
   const uint32_t pair = blockIdx.x;
   if (!p.pair_ok[pair]) return;
-  const float *h = p.h32 + (size_t)pair * p.d_ff;
+  uint32_t *hg = p.hg + (size_t)pair * p.hblocks * kGroupRecDwords;
+  const float *h = reinterpret_cast<const float *>(hg);
   if constexpr (MODE == kF16Pair) {
-    quant_vector<FMT>(h, p.hblocks, reinterpret_cast<uint4 *>(p.hg) + (size_t)pair * p.hblocks * 8, p.hs + pair);
+    quant_vector<FMT>(h, p.hblocks, reinterpret_cast<uint4 *>(hg), p.hs + pair);
   } else {
     // whole quads of lanes per block; d_ff / 8 groups are a multiple of 8
     for (uint32_t g = threadIdx.x; g < p.hblocks * 4; g += blockDim.x) {
-      const size_t b = (size_t)pair * p.hblocks + g / 4;
       float v[8];
       load_group<FMT>(h, g / 4, g % 4, v);
-      quant_group_q8(v, reinterpret_cast<uint4 *>(p.hg) + b * 4 + g % 4, p.hs + b, g % 4, true);
+      quant_group_q8(v, reinterpret_cast<uint4 *>(hg) + (size_t)(g / 4) * 8, g % 4, true);  // after the quad's loads
     }
   }
 }

@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "mer_device.hpp"
+#include "mer_grouped_plan.hpp"
 
 namespace mer {
 
@@ -160,18 +161,6 @@ struct DecodeParams {
 };
 
 // ---- grouped multi-token path (mer_grouped.hip) --------------------------
-constexpr uint32_t kMaxGroupedExperts = 4096;  // table entries the grouping kernel counts in LDS
-constexpr uint32_t kMaxGroupedPairs = 4096;    // routed (token, slot) pairs per call
-
-// Input formats of the projection kernels (mer_grouped.hip).
-enum GroupMode : uint32_t { kGroupDigits = 0, kGroupQ8Act = 1, kGroupF16Pair = 2 };
-
-struct GroupTile {
-  const uint8_t *blob;  // the expert's blob
-  uint32_t start;       // first pair of the tile in plist
-  uint32_t count;       // pairs in the tile: 1..16 (kGroupDigits) or 1..64
-};
-
 struct GroupedParams {
   const void *const *table;
   uint32_t table_len;
@@ -186,8 +175,8 @@ struct GroupedParams {
   float swiglu_limit;        // gate clamp before SiLU (+inf = none)
   size_t proj_bytes;
   // scratch
-  uint32_t *xg;              // x records [n_tok][xblocks][4 k-groups], 8 dwords each (4 under kGroupQ8Act)
-  uint32_t *hg;              // h records [n_pairs][hblocks][4]
+  uint32_t *xg;              // x records [n_tok][xblocks][kGroupRecDwords]
+  uint32_t *hg;              // h records [n_pairs][hblocks][kGroupRecDwords]; f16 modes: first f32 h [n_pairs][d_ff]
   float *partial;            // w_i y_i [n_parts][n_pairs][d_model]
   uint32_t *plist;           // pairs grouped by expert [n_pairs]
   uint32_t *pair_ok;         // [n_pairs] 1 = routed to a resident expert with a nonzero weight
@@ -196,8 +185,7 @@ struct GroupedParams {
   uint32_t *status;
   uint32_t mode;             // kGroupDigits, kGroupQ8Act or kGroupF16Pair
   uint32_t n_parts, part_blocks;  // K parts of the down projection, blocks of each
-  float *xs, *hs;            // f16 modes: the scales of the records, per vector or (kGroupQ8Act) per block
-  float *h32;                // f16 modes: f32 h [n_pairs][d_ff]
+  float *xs, *hs;            // kGroupF16Pair: the vectors' scales [n_tok], [n_pairs]
 };
 
 size_t grouped_group_lds_bytes(uint32_t table_len, uint32_t n_pairs);
