@@ -146,8 +146,13 @@ __global__ __launch_bounds__(kRouterThreads) void router_logits_kernel(RouterPar
 // logits instead of once per logit or per four.  Stages of 128 k-indices go
 // through LDS, read whole rows at a time: rows of a power-of-two length start
 // in one L2 channel and one L1 set, so 16 rows per load instruction (straight
-// from the operand layout) ran at a third of the rate; for the same reason
-// each workgroup starts at another stage.  Wave w takes the stage's run w of
+// from the operand layout) ran at a third of the rate.  Every workgroup takes
+// the stages in the same order, so a logit does not depend on the tile that
+// its token and its expert fall in and equal gate rows tie exactly (starting
+// each workgroup at another stage gains nothing: 128 experts x 2048, 2048
+// tokens 24.3 us, 24.5 in order; 256 x 7168, 2048 tokens 90 and 86).  Another
+// order than the kernel above, so a call on either side of the choice between
+// them differs in the last bits.  Wave w takes the stage's run w of
 // 16 k-indices; lane l holds four consecutive elements of row l % 16
 // (k-indices 4 (l / 16) .. + 3 of the run), one for each of four products,
 // which is the same permutation of k on both sides.  Sums are kept short, as
@@ -173,14 +178,14 @@ __global__ __launch_bounds__(64 * kRouterMWaves) void router_logits_mfma_kernel(
       const_cast<float *>(p.gate + (size_t)e0 * p.d_model), 0, ne * p.d_model * 4u, 0x00020000);
   const uint32_t srow = threadIdx.x / 32, scol = 4 * (threadIdx.x % 32);
   const uint32_t stages = (p.d_model + kRouterStage - 1) / kRouterStage;
-  uint32_t next = q % stages;
+  uint32_t next = 0;
   struct Buf {
     v4f v[4];
     uint32_t k;
   };
   auto load = [&](Buf &b) {
     b.k = kRouterStage * next + scol;
-    next = next + 1 == stages ? 0u : next + 1;
+    ++next;  // loads past the last stage read zeros
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) {
       const uint32_t o = b.k < p.d_model ? ((srow + 16 * (j % 2)) * p.d_model + b.k) * 4u : 0x80000000u;
@@ -207,8 +212,7 @@ __global__ __launch_bounds__(64 * kRouterMWaves) void router_logits_mfma_kernel(
   store(buf[0], 0);
   load(buf[0]);
   __syncthreads();
-  // stage s is in slab s % 2, s + 1 and s + 2 in buf (loads past the last
-  // stage repeat the first ones and are not used)
+  // stage s is in slab s % 2, s + 1 and s + 2 in buf
   for (uint32_t s = 0; s < stages; s += 2) {
 #pragma unroll
     for (uint32_t u = 0; u < 2; ++u) {

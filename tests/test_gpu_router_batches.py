@@ -41,3 +41,24 @@ def test_router_batches(mer, oracle, gpu, n_experts, d_model, top_k, opts, n_tok
         assert list(ids[t][:len(want_ids)]) == list(want_ids), f"ids token {t}"
         assert (ids[t][len(want_ids):] == -1).all()
         assert np.allclose(ws[t][:len(want_ws)], want_ws, rtol=1e-5, atol=1e-7), f"weights token {t}"
+
+
+@pytest.mark.parametrize("d_model", [64, 200, 384, 1031, 2048, 7168])
+def test_equal_rows_have_equal_logits(mer, gpu, d_model):
+    """A logit depends on its token and its gate row alone, not on the tile
+    that they fall in: copies of a token, and experts with the same gate row,
+    get the same bits, so their ties go to the lower id in every tile."""
+    say(f"router equal rows dm={d_model}")
+    r = routing(mer)
+    rng = np.random.default_rng(d_model)
+    n_tok, n_experts, period = 1030, 99, 33
+    base_w = (rng.standard_normal((period, d_model)) * 0.05).astype(np.float32)
+    base_x = rng.standard_normal((5, d_model)).astype(np.float32)
+    w, x = np.tile(base_w, (n_experts // period, 1)), np.tile(base_x, (n_tok // 5, 1))
+    ids, ws, lg = r.route_linear_gate_gpu(dev(w, gpu), dev(x, gpu), 3, return_logits=True)
+    ids, ws, lg = ids.cpu().numpy(), ws.cpu().numpy(), lg.cpu().numpy()
+    want = lg[:5, :period]
+    assert (lg.reshape(-1, 5, n_experts // period, period) == want[None, :, None, :]).all()
+    best = want.argmax(1)
+    assert (ids.reshape(-1, 5, 3) == best[None, :, None] + period * np.arange(3)).all()
+    assert (ws.reshape(-1, 5, 3) == ws[:5]).all()
