@@ -848,7 +848,7 @@ int run_grouped(Workspace &w, int dtype, size_t dm, size_t dff, uint32_t n_token
   p.hblocks = (uint32_t)(dff / 32);
   p.proj_bytes = div_ceil(dm * dff, 32) * block_bytes(dtype);
   p.status = dev.status;
-  GroupedPlan pl = plan_grouped(p.q8act != 0, dm, dff, n_tokens, top_k, table_len);
+  GroupedPlan pl = plan_grouped(fmt_of(dtype) == FMT_Q4_0, p.q8act != 0, dm, dff, n_tokens, top_k, table_len);
   float *f = nullptr;
   int rc = ensure_scratch_upto(w, pl.need, pl.want, &f);
   if (rc) return rc;

@@ -25,7 +25,7 @@ def _call(gpu, dtype, dm, dff, n_tok, k, table_len, blob):
 
 @pytest.mark.parametrize("dtype,dm,dff,large,small", [
     # 256 x 8 pairs over 140 experts (tiles of 16), then 250 x 8 over 8 (tiles of 64)
-    (5, 256, 1792, (256, 8, 140), [(250, 8, 8), (256, 8, 8), (17, 1, 1)]),
+    (5, 1024, 1792, (256, 8, 140), [(250, 8, 8), (256, 8, 8), (17, 1, 1)]),
     # down projection in one part, then in two
     (4, 16384, 4160, (1792, 1, 8), [(1728, 1, 8), (1024, 1, 2), (40, 1, 1)]),
 ])
