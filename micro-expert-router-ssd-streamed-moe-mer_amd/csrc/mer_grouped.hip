@@ -740,15 +740,20 @@ __device__ __forceinline__ v8h unpack_q8(uint32_t lo, uint32_t hi) {
 // Asynchronous copy of 16 bytes per lane from a buffer (an offset past its
 // end reads zeros) to LDS at `lds` + 16 * lane.  The compiler does not see
 // it: the caller waits (wait_vm) before the barrier that publishes it.  M0
-// holds the LDS address; s_nop: wait states between a write of M0 or of a
-// resource word and its use.
+// holds the LDS address and is named as written, so the compiler does not
+// take an earlier value of its own to be still there (the warning that it does
+// not save M0 across the statement is beside the point); s_nop: wait states
+// between a write of M0 or of a resource word and its use.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void async_lds16(v4u rsrc, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds) : "memory", "m0");
 }
 // The same for 4 bytes per lane, to LDS at `lds` + 4 * lane.
 __device__ __forceinline__ void async_lds4(v4u rsrc, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // Wait until at most N of this wave's vector memory operations are in flight.
 template <int N>
 __device__ __forceinline__ void wait_vm() {
