@@ -72,6 +72,7 @@
 // to LDS as they are and become f16 in registers.
 #include <type_traits>
 
+#include "../../include/mer_hip.h"
 #include "mer_internal.hpp"
 
 namespace mer {
@@ -195,11 +196,13 @@ __device__ __forceinline__ constexpr uint32_t kgroup_elem(uint32_t m, int i) {
   }
 }
 
-// One k-group of a Q8_0-activation record (the four groups' 16 bytes, then
-// the block's f32 scale): 8 elements (in kgroup_elem order) of a block whose
-// 4 groups sit in 4 adjacent lanes (lane & 3 = group m).  Only lanes with
-// `store` write.
-__device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint4 *rec, uint32_t m, bool store) {
+// One k-group of a vector's Q8_0 activation: 8 elements (in kgroup_elem
+// order) of a block whose 4 groups sit in 4 adjacent lanes (lane & 3 = group
+// m).  `vec`: the vector's region of kRecBytes a block; its first half takes
+// the blocks' records (four groups of 16 bytes), the second their f32 scales,
+// so a cache line holds two records.  Only lanes with `store` write.
+__device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint32_t *vec, uint32_t blocks, uint32_t b, uint32_t m,
+                                               bool store) {
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[i]));
@@ -210,8 +213,8 @@ __device__ __forceinline__ void quant_group_q8(const float (&v)[8], uint4 *rec, 
   v8h q;
 #pragma unroll
   for (int i = 0; i < 8; ++i) q[i] = (_Float16)quantize_elem_q8(v[i], bs.inv);
-  rec[m] = __builtin_bit_cast(uint4, q);
-  if (m == 0) *reinterpret_cast<float *>(rec + 4) = bs.s;
+  reinterpret_cast<uint4 *>(vec)[(size_t)b * 4 + m] = __builtin_bit_cast(uint4, q);
+  if (m == 0) reinterpret_cast<float *>(vec)[(size_t)blocks * (kGroupRecDwords / 2) + b] = bs.s;
 }
 
 // Eight elements of block b, k-group m of the f32 vector x, in kgroup_elem order.
@@ -297,7 +300,7 @@ __global__ __launch_bounds__(1024) void group_kernel(GroupedParams p) {
       float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if constexpr (MODE == kQ8Act) {
         if (valid) load_group<FMT>(p.x, tb, m, v);
-        quant_group_q8(v, reinterpret_cast<uint4 *>(p.xg) + (size_t)tb * 8, m, valid);
+        quant_group_q8(v, p.xg + (size_t)(tb / p.xblocks) * p.xblocks * kGroupRecDwords, p.xblocks, tb % p.xblocks, m, valid);
       } else {
         if (valid) load_group<FMT_Q8_0>(p.x, tb, m, v);  // eight consecutive elements
         quant_group(v, p.xg + ((size_t)tb * 4 + m) * kGRec, valid, p.q8act != 0);
@@ -814,13 +817,14 @@ constexpr uint32_t kBigStride = 16 * kBigGran;
 constexpr uint32_t kBigSlab = kBigRows * kBigStride;
 constexpr uint32_t kXSlots = 5;
 constexpr uint32_t kX0 = 2 * kBigSlab;                    // LDS offset of the input slots
-constexpr uint32_t kRecBytes = 4 * kGroupRecDwords;       // a block's record in memory
+constexpr uint32_t kRecBytes = 4 * kGroupRecDwords;       // a block of a vector's inputs in memory
 // LDS bytes of a block of 64 pairs' inputs: records, or records and scales
 template <int MODE> constexpr uint32_t kXSlot = MODE == kF16Pair ? 64 * 128 : 64 * 64 + 4 * 256;
 
 template <int FMT, int MODE, bool FUSED, int NG>
 struct GBig {
   static constexpr int kParts = MODE == kF16Pair ? 2 : 1;  // f16 parts of an input
+  static constexpr uint32_t kRec = 64u * kParts;           // bytes of a block's record
   static constexpr uint32_t kBB = FmtTraits<FMT>::kBlockBytes;
   static constexpr int kSB = FMT == FMT_Q4_0 ? 4 : 2;      // blocks per stage: 72 or 68 of 80 bytes
   static constexpr int kNW = (int)(kBigRows * kBigGran / 256);  // weight copies per wave and stage
@@ -888,9 +892,9 @@ struct GBig {
       const uint32_t n = 16 * (i / kParts) + lane % 16;
       const uint32_t pair = n < count ? p.plist[start + n] : 0u;
       // a column without a pair reads zeros
-      const uint32_t rec = (FUSED ? pair / p.top_k : pair) * vec_bytes + b0 * kRecBytes;
-      xoff[j] = n < count ? rec + 64u * (i % kParts) + 16u * (lane / 16) : kNoLoad;
-      if (MODE == kQ8Act && n < count) soff = rec + 64u;
+      const uint32_t vec = (FUSED ? pair / p.top_k : pair) * vec_bytes;
+      xoff[j] = n < count ? vec + b0 * kRec + 64u * (i % kParts) + 16u * (lane / 16) : kNoLoad;
+      if (MODE == kQ8Act && n < count) soff = vec + row_blocks * kRec + b0 * 4u;
     }
     uint32_t x_issued = 0, x_slot = 0;
     auto issue_x = [&]() {
@@ -898,11 +902,11 @@ struct GBig {
 #pragma unroll
       for (int j = 0; j < kXCopies; ++j) {
         async_lds16(xr, xoff[j] | none, lds0 + kX0 + x_slot * kXSlot<MODE> + (wave + 4u * j) % (2 * NG * kParts) * 1024u);
-        xoff[j] += kRecBytes;
+        xoff[j] += kRec;
       }
       if constexpr (MODE == kQ8Act) {  // the scales of the copy's 16 vectors, four times over
         async_lds4(xr, soff | none, lds0 + kX0 + x_slot * kXSlot<MODE> + 4096u + wave % (2 * NG) * 256u);
-        soff += kRecBytes;
+        soff += 4u;
       }
       ++x_issued;
       x_slot = x_slot + 1 == kXSlots ? 0u : x_slot + 1;
@@ -1131,11 +1135,22 @@ __global__ __launch_bounds__(256) void hquant_kernel(GroupedParams p) {
   if constexpr (MODE == kF16Pair) {
     quant_vector<FMT>(h, p.hblocks, reinterpret_cast<uint4 *>(hg), p.hs + pair);
   } else {
-    // whole quads of lanes per block; d_ff / 8 groups are a multiple of 8
-    for (uint32_t g = threadIdx.x; g < p.hblocks * 4; g += blockDim.x) {
-      float v[8];
-      load_group<FMT>(h, g / 4, g % 4, v);
-      quant_group_q8(v, reinterpret_cast<uint4 *>(hg) + (size_t)(g / 4) * 8, g % 4, true);  // after the quad's loads
+    // All of h goes to registers before its place takes the records, which
+    // lie closer together.  Whole quads of lanes per block: d_ff / 8 groups
+    // are a multiple of 8.
+    constexpr int kMax = MER_MAX_EXPERT_DIM / 8 / 256;
+    const uint32_t groups = p.hblocks * 4;
+    float v[kMax][8];
+#pragma unroll
+    for (int j = 0; j < kMax; ++j) {
+      const uint32_t g = threadIdx.x + 256u * j;
+      if (g < groups) load_group<FMT>(h, g / 4, g % 4, v[j]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kMax; ++j) {
+      const uint32_t g = threadIdx.x + 256u * j;
+      if (g < groups) quant_group_q8(v[j], hg, p.hblocks, g / 4, g % 4, true);
     }
   }
 }

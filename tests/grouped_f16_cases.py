@@ -22,6 +22,7 @@ LONG_ROWS_QMM = [
     (Q4, 1, 192, 8256, 65, 1, 1, 4),
     (Q4, 1, 576, 8256, 40, 1, 1, 4),
     (Q4, 1, 128, 8256, 40, 2, 2, 4),
+    (Q4, 1, 64, 16384, 33, 1, 1, 4),    # the longest rows
 ]
 # many experts: the sums in one part or two
 MANY = [
