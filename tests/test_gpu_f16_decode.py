@@ -13,12 +13,20 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from test_gpu_decode_geometry import SHAPES as VARIANTS  # noqa: E402
+from test_gpu_decode_geometry import _plan  # noqa: E402
 from test_gpu_parity import Q4, Q8, _table, make_expert, randn, say, to_dev  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(Q4, 64, 64, 1), (Q8, 64, 128, 3), (Q4, 192, 320, 5), (Q8, 576, 64, 2), (Q4, 1024, 5120, 2), (Q4, 2048, 768, 8),
           (Q8, 2048, 768, 9), (Q8, 4160, 128, 4)]
+# every instance of the kernel's f16 mode, by format, lane groups and pairing
+SHAPES += [(dt, dm, dff, n * k) for dt in (Q4, Q8) for dm, dff, n, k in VARIANTS]
+
+
+def test_shapes_reach_every_variant():
+    assert {_plan(dm, dff, n * k, 1) for dm, dff, n, k in VARIANTS} == set(VARIANTS.values())
 
 
 @pytest.mark.parametrize("dtype,dm,dff,n", SHAPES)

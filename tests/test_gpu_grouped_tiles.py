@@ -1,7 +1,8 @@
-"""The grouped path's 64-pair tiles (f16 MFMA) at the sizes where they can go
-wrong, against the CPU oracle: tiles of one to several 16-pair groups, K that
-ends inside a stage, rows that end inside a row tile, the down projection in
-K parts, and the call sizes on either side of the kernel choice."""
+"""The grouped path at the ends of its tiles, against the CPU oracle: tiles
+of one to several 16-pair groups, K that ends inside a stage, rows that end
+inside a row tile, and the grouping of pairs.  These calls are small: most run
+the int8 kernel's tiles of 16 pairs, those with 8256 inner rows the f16
+kernel's tiles of 64, which test_gpu_grouped_f16.py covers."""
 from __future__ import annotations
 
 import numpy as np
@@ -23,15 +24,16 @@ def _routes(n_tok, k, n_exp, seed):
 
 
 @pytest.mark.parametrize("dtype,dm,dff,n_exp,n_tok,k", [
-    (Q4, 64, 64, 1, 16, 1),      # half a stage of K, one 16-pair group
-    (Q8, 64, 64, 1, 33, 1),      # one stage, a tile of 33 pairs
-    (Q8, 192, 320, 2, 65, 1),    # a tile more than 64 pairs need; row tiles of 128 and 256 rows cut short
-    (Q4, 192, 320, 3, 48, 2),    # six and ten blocks of K: stages of four cut short
-    (Q4, 576, 192, 2, 40, 2),    # eighteen blocks: one partial sum of sixteen and a rest
-    (Q8, 1088, 64, 1, 17, 1),    # 34 blocks, seventeen stages
-    (Q4, 64, 4160, 2, 17, 2),    # down K of 130 blocks in two parts, 68 + 62
-    (Q8, 128, 8256, 1, 20, 1),   # 258 blocks in four parts, the last one short
-    (Q8, 64, 64, 140, 300, 7),   # 15 pairs per expert: the int8 kernel's 128-row gate/up
+    (Q4, 64, 64, 1, 16, 1),      # two blocks of K, one 16-pair group
+    (Q8, 64, 64, 1, 33, 1),      # two full tiles and one pair
+    (Q8, 192, 320, 2, 65, 1),    # d_model that no 128-row tile divides
+    (Q4, 192, 320, 3, 48, 2),    # six and ten blocks of K: stages cut short
+    (Q4, 576, 192, 2, 40, 2),    # eighteen blocks
+    (Q8, 1088, 64, 1, 17, 1),    # 34 blocks, one pair past a tile
+    (Q4, 64, 4160, 2, 17, 2),    # down K of 130 blocks
+    (Q8, 128, 8256, 1, 20, 1),   # f16 tiles: 258 blocks in four parts, the last one short
+    (Q4, 64, 64, 140, 300, 7),   # 2100 pairs: 128-row gate/up workgroups
+    (Q8, 64, 64, 140, 300, 7),   # 2100 pairs: 128-row gate/up workgroups
 ])
 def test_tiles_vs_oracle(mer, oracle, gpu, dtype, dm, dff, n_exp, n_tok, k):
     say(f"grouped tiles dtype={dtype} dm={dm} dff={dff} experts={n_exp} tokens={n_tok} k={k}")
@@ -51,6 +53,7 @@ def test_tiles_vs_oracle(mer, oracle, gpu, dtype, dm, dff, n_exp, n_tok, k):
 
 @pytest.mark.parametrize("dm,dff,n_exp,n_tok,k", [
     (64, 64, 1, 16, 1), (192, 320, 2, 70, 1), (128, 4160, 2, 33, 1), (576, 192, 1, 64, 1),
+    (64, 64, 140, 300, 7),  # 2100 pairs: 128-row gate/up workgroups
 ])
 def test_tiles_qmm_vs_oracle(mer, oracle, gpu, dm, dff, n_exp, n_tok, k):
     say(f"grouped tiles qmm dm={dm} dff={dff} experts={n_exp} tokens={n_tok} k={k}")
