@@ -303,9 +303,9 @@ int mer_hip_expert_batch_f16(int dtype, size_t d_model, size_t d_ff, size_t n_ex
  * zero-weight slots skipped, misses recorded in the device status -- but
  * the routed (token, slot) pairs are grouped by expert on the device, so
  * every expert's weights are read once per tile of its tokens and the
- * projections run as MFMA contractions: int8 over tiles of 16 pairs where
- * experts have few, f16 over tiles of 64 where they have 16 or more on
- * average (8 for many large experts).  This is the batched counterpart of
+ * projections run as MFMA contractions: int8 over tiles of 16 pairs, or f16
+ * over tiles of 64 where the call has 16 or more pairs per table entry (8 for
+ * many large Q4_0 experts) and work enough to fill the chip with them.  This is the batched counterpart of
  * routed_expert_matmul_batch_q4 (backend/mod.rs:4401-4418) and of the
  * per-pair dispatch loop of forward_moe_resident_cpu (engine.rs:1761-1848)
  * over a prefill batch.  Requires d_model and d_ff to be multiples of 64,
@@ -313,7 +313,8 @@ int mer_hip_expert_batch_f16(int dtype, size_t d_model, size_t d_ff, size_t n_ex
  * block fixed point (int8; error <= 2^-24 of each 32-element block's
  * maximum) or as pairs of f16 with one power-of-two scale per vector (error
  * <= 2^-23 of each element, or 2^-39 of the vector's maximum where that is
- * more). */
+ * more: beside an outlier of more than 2^15 times its block's largest element
+ * an element keeps fewer bits than in the block fixed point). */
 int mer_hip_moe_grouped(int dtype, size_t d_model, size_t d_ff,
                         size_t n_tokens, size_t top_k,
                         const void *const *d_expert_table, size_t table_len,

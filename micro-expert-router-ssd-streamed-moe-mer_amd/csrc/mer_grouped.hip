@@ -1,7 +1,7 @@
 // mer_grouped.hip -- grouped per-expert path for multi-token batches (gfx950).
 //
 // A prefill-sized batch routes many tokens to the same expert, so each
-// expert's weights can be read once for all of its tokens.  That turns
+// expert's weights can be read once per tile of its tokens.  That turns
 // the per-expert work into a real dense contraction: [rows x K] weights by
 // [K x tokens], run on MFMA one GGUF block (K = 32) at a
 // time.  Reference semantics are those of the decode path: every
@@ -21,7 +21,7 @@
 //                  w_i * y_i per pair
 //   combine_kernel out[t] = [x +] sum over slots in slot order
 //
-// Two projection kernels, by the pairs an expert has on average (run_grouped):
+// Two projection kernels, by the sizes of the call (mer_grouped_plan.hpp):
 //   gproj  int8 MFMA, tiles of 16 pairs, for few pairs, where streaming the
 //          weights is everything;
 //   gbig   f16 MFMA, tiles of 64 pairs.
@@ -44,7 +44,8 @@
 // puts its largest element in [2^14, 2^15), hi the f16 nearest to x / S and
 // lo the f16 nearest to the rest: an error of at most 2^-23 |x|, and 2^-39 of
 // the vector's largest element where lo underflows (elements below 2^-16 of
-// it).  Per block two chained products, lo first, give sum q (hi + lo) in
+// it): beside an outlier of more than 2^15 times its own block's largest
+// element, an input keeps fewer bits than in gproj.  Per block two chained products, lo first, give sum q (hi + lo) in
 // f32; times d_w it goes to an f32 accumulator.  The matrix unit rounds its
 // sums towards minus infinity, a bias that would grow with the number of
 // blocks, so every other block carries both its weights and its scale
@@ -709,6 +710,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGWavesPerE
 // ---- gbig: tiles of up to 64 pairs, shared parts ---------------------------
 
 // f16 weights of one MFMA k-group from its raw bytes (exact integers).
+// The widely published bit trick: 0x6400 | n is 1024 + n, since an ulp of
+// [1024, 2048) is 1.
 // Q4_0: qs dword -> q - 8 of bytes' low and high nibbles, in kgroup_elem
 // order: (1024 + n) - 1032, and (1024 + 16 n) / 16 - 72 for high nibbles.
 // NEG: the negated weights.
@@ -803,12 +806,12 @@ __device__ __forceinline__ bool group_item(const GroupedParams &p, uint32_t row_
 // product holds weight row l % 32 and pairs 8 (i / 4) + 4 (l / 32) + i % 4.
 //
 // Bound: matrix unit and vector issue slots at the clock the power limit
-// leaves (Mixtral Q4_0, 4096 pairs: 1.8 GHz, 49% and 59% of cycles busy; the
-// two f16 products alone take 1.4 ms of the gate/up launch's 2.15 at the
+// leaves (Mixtral Q4_0, 4096 pairs: 1.74 GHz, 49% and 63% of cycles busy; the
+// two f16 products alone take 1.4 ms of the gate/up launch's 2.04 at the
 // rate the unit sustains on such data).  One product of a wave's own has to
 // saturate the unit while its other wave works on sums, which 32 x 32 tiles
 // do and 16 x 16 tiles do not.  Mixtral Q4_0 top-2, 2048 tokens, against the
-// int8 kernel: gate/up 4.49 -> 2.15 ms, down 2.16 -> 1.1 ms; 333 tokens under
+// int8 kernel: gate/up 4.49 -> 2.04 ms, down 2.16 -> 1.09 ms; 333 tokens under
 // MER_MOE_QMM 0.84 -> 0.46 and 0.42 -> 0.24 ms (its products are half as many,
 // its sums carry a scale per pair as well: vector issue).
 constexpr uint32_t kBigRows = 256;

@@ -260,8 +260,8 @@ def moe_grouped(dtype: WeightDtype, d_model: int, d_ff: int, table: torch.Tensor
                 residual: bool = False, accumulate: bool = False, qmm: bool = False) -> torch.Tensor:
     """moe_forward for a multi-token batch on the grouped MFMA path:
     pairs grouped by expert on the device, each expert's weights read once
-    for all of its tokens (the batched routed_expert_matmul_batch_q4,
-    backend/mod.rs:4401-4418).  Same arguments and combine as moe_forward;
+    per tile of 16 or 64 of its tokens (the batched
+    routed_expert_matmul_batch_q4, backend/mod.rs:4401-4418).  Same arguments and combine as moe_forward;
     qmm: Q4_0 experts with Candle's QMatMul arithmetic (MER_MOE_QMM)."""
     _init_for(x)
     n_tokens, top_k = expert_ids.shape
